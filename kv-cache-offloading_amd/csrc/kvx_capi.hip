@@ -185,9 +185,9 @@ static int run_batches(bool save, void* pool, const kvx_block_layout* layout, in
       b.ids[i] = ids[base + i];
       b.entries[i] = entries[base + i];
     }
-    const bool vec = vector_access_ok(pool, *layout, b.entries, b.n);
-    hipError_t err = save ? launch_save(pool, *layout, format, b, scale_offset, vec, 0, stream)
-                          : launch_restore(pool, *layout, format, b, scale_offset, vec, 0, stream);
+    const Access access = access_of(pool, *layout, b.entries, b.n);
+    hipError_t err = save ? launch_save(pool, *layout, format, b, scale_offset, access, 0, stream)
+                          : launch_restore(pool, *layout, format, b, scale_offset, access, 0, stream);
     if (err != hipSuccess) return hip_status(err, save ? "save kernel launch" : "restore kernel launch");
   }
   return KVX_OK;
@@ -225,8 +225,8 @@ static int token_copy(bool gather, void* pool, const kvx_block_layout* l, const 
       b.entries[i] = (uint64_t)(uintptr_t)dense + (uint64_t)((base + i) * plane_bytes);
     }
     const int64_t last = base + b.n == nblocks ? tail_bytes : plane_bytes;
-    const bool vec = vector_access_ok(pool, *l, b.entries, b.n);
-    hipError_t err = launch_token_copy(gather, pool, *l, b, vec, dense_plane_stride, last, stream);
+    const Access access = access_of(pool, *l, b.entries, b.n);
+    hipError_t err = launch_token_copy(gather, pool, *l, b, access, dense_plane_stride, last, stream);
     if (err != hipSuccess) return hip_status(err, gather ? "token gather launch" : "token scatter launch");
   }
   return KVX_OK;
@@ -265,6 +265,8 @@ static int token_fp8(bool gather, void* pool, const kvx_block_layout* l, const i
   // Vector kernels store scales 16 bytes at a time from tile-aligned rows.
   const bool aligned = p0 % 16 == 0 && s0 % 16 == 0 && (num_rows * hd) % 16 == 0 && (num_rows * sb) % 16 == 0 &&
                        (R * sb) % 16 == 0;
+  // 8-byte pieces need every plane's payload to start on 8 bytes.
+  const bool pieces = (num_rows * hd) % 8 == 0;
   TokenSpan span{num_rows * hd, num_rows * sb, R * (sb - hd), (int32_t)R};
   BlockBatch b;
   for (int64_t base = 0; base < nblocks; base += kMaxBatch) {
@@ -276,8 +278,9 @@ static int token_fp8(bool gather, void* pool, const kvx_block_layout* l, const i
     span.last_rows = (int32_t)(base + b.n == nblocks ? num_rows - (nblocks - 1) * R : R);
     // Entry i's scales: scales + (base + i) * R * sb = entries[i] + scale_offset + i * scale_entry_step.
     const int64_t scale_offset = (int64_t)(s0 + (uintptr_t)(base * R * sb)) - (int64_t)(p0 + (uintptr_t)(base * R * hd));
-    const bool vec = aligned && vector_access_ok(pool, *l, b.entries, b.n);
-    hipError_t err = launch_token_fp8(gather, pool, *l, b, scale_offset, span, vec, stream);
+    Access access = access_of(pool, *l, b.entries, b.n);
+    if (!aligned) access = std::min(access, pieces ? kPieceAccess : kAnyAccess);
+    hipError_t err = launch_token_fp8(gather, pool, *l, b, scale_offset, span, access, stream);
     if (err != hipSuccess) return hip_status(err, gather ? "FP8 token gather launch" : "FP8 token scatter launch");
   }
   return KVX_OK;
@@ -663,9 +666,9 @@ struct kvx_cache {
       b.ids[i] = ids[i];
       b.entries[i] = (uint64_t)(uintptr_t)(staging ? staging + (int64_t)i * entry_stride : host_entry(slots[i]));
     }
-    const bool vec = vector_access_ok(pool, layout, b.entries, b.n);
-    hipError_t err = save ? launch_save(pool, layout, format, b, scale_offset, vec, staging ? 0 : direct_save_grid(), s)
-                          : launch_restore(pool, layout, format, b, scale_offset, vec,
+    const Access access = access_of(pool, layout, b.entries, b.n);
+    hipError_t err = save ? launch_save(pool, layout, format, b, scale_offset, access, staging ? 0 : direct_save_grid(), s)
+                          : launch_restore(pool, layout, format, b, scale_offset, access,
                                            staging ? 0 : direct_restore_grid(), s);
     return hip_status(err, save ? "save kernel launch" : "restore kernel launch");
   }
@@ -898,7 +901,7 @@ int kvx_cache_create(void* pool, const kvx_block_layout* layout, int32_t format,
   c->split = save_stream != restore_stream;
   // Host slots are 256-byte aligned and entry_stride apart (a multiple of 256),
   // so the pool alone decides whether the vector kernels can address them.
-  c->host_reads_ok = striding_restore_supported(*layout, format, vector_access_ok(pool, *layout, nullptr, 0));
+  c->host_reads_ok = striding_restore_supported(*layout, format, access_of(pool, *layout, nullptr, 0));
   c->pending_save.assign(layout->num_blocks, nullptr);
   c->pending_restore.assign(layout->num_blocks, nullptr);
   DeviceScope scope;

@@ -59,34 +59,39 @@ int hip_status(hipError_t err, const char* what);
 
 int check_layout(const kvx_block_layout* layout, int32_t format);
 
+// What a pool and its entries' addresses allow. The pool's base and strides
+// are multiples of 16 bytes for the last two, and the entries of 16
+// (kVectorAccess: the tiled kernels) or of 8 (kPieceAccess: FP8 payloads
+// written and read 8 codes at a time, scales one at a time). kAnyAccess runs
+// the element-granular kernels.
+enum Access { kAnyAccess, kPieceAccess, kVectorAccess };
+
 // Kernel launchers: arguments are validated by the caller.
-// `vector_ok`: the pool base, both strides and every entry allow 16-byte
-// vector access; otherwise the element-granular kernels run.
 // `max_grid` > 0 caps a vector kernel's workgroups (they then stride over
 // the tiles): for saves written to and restores read from host memory, which
 // hold their workgroups while the bytes cross the host link.
 hipError_t launch_save(const void* pool, const kvx_block_layout& layout, int32_t format,
-                       const BlockBatch& batch, int64_t scale_offset, bool vector_ok, int32_t max_grid,
+                       const BlockBatch& batch, int64_t scale_offset, Access access, int32_t max_grid,
                        hipStream_t stream);
 hipError_t launch_restore(void* pool, const kvx_block_layout& layout, int32_t format,
-                          const BlockBatch& batch, int64_t scale_offset, bool vector_ok, int32_t max_grid,
+                          const BlockBatch& batch, int64_t scale_offset, Access access, int32_t max_grid,
                           hipStream_t stream);
 // True when a restore launched with max_grid > 0 runs the striding kernel,
 // whose reads of host entries are system-scope loads (the element-granular
 // kernels read with plain loads and must not read host memory).
-bool striding_restore_supported(const kvx_block_layout& layout, int32_t format, bool vector_ok);
+bool striding_restore_supported(const kvx_block_layout& layout, int32_t format, Access access);
 // Token gather/scatter between a sequence's blocks and a dense
 // [planes][rows][head_dim] buffer: entries are the dense buffer at
 // block_index * plane_bytes, dense_plane_stride apart per plane, and the
 // batch's last block copies last_bytes per plane.
 hipError_t launch_token_copy(bool gather, void* pool, const kvx_block_layout& layout, const BlockBatch& batch,
-                             bool vector_ok, int64_t dense_plane_stride, int64_t last_bytes, hipStream_t stream);
+                             Access access, int64_t dense_plane_stride, int64_t last_bytes, hipStream_t stream);
 // The same with FP8 quantisation (gather) or dequantisation (scatter):
 // entries are the payload rows of each block, scales per `span`.
 hipError_t launch_token_fp8(bool gather, void* pool, const kvx_block_layout& layout, const BlockBatch& batch,
-                            int64_t scale_offset, const TokenSpan& span, bool vector_ok, hipStream_t stream);
-// True when 16-byte vector kernels may address this pool/entry combination.
-bool vector_access_ok(const void* pool, const kvx_block_layout& layout, const uint64_t* entries, int32_t n);
+                            int64_t scale_offset, const TokenSpan& span, Access access, hipStream_t stream);
+// The widest access this pool/entry combination allows.
+Access access_of(const void* pool, const kvx_block_layout& layout, const uint64_t* entries, int32_t n);
 hipError_t launch_store_kvcache(const void* key, int64_t key_stride, const void* value,
                                 int64_t value_stride, void* k_cache, void* v_cache,
                                 const int32_t* slot_mapping, int64_t num_tokens, int64_t row_elems,

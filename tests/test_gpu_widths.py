@@ -1,0 +1,105 @@
+"""The kernels for rows of any width at the edges of their tiles, against the oracle (bit-exact)."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import bf16_bits, bf16_tensor, finite_bf16_rows, u8
+from kvx import ops
+from oracle import kvx_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+
+SCALES = [torch.float32, torch.bfloat16]
+
+
+def finite_pool(gpu, layers, blocks, bs, heads, hd, seed=0):
+    shape = (2, layers, blocks, bs, heads, hd)
+    return bf16_tensor(finite_bf16_rows(int(np.prod(shape[:-1])), hd, seed), gpu).view(shape)
+
+
+# (layers, block tokens, heads, head_dim). A save tile holds at most 768 8-element pieces, cut to whole rows (64 rows
+# of 96, 72 of 80, 48 of 112 and of 128); a restore tile 512 pieces. Rows of 8 are one piece, rows of 6144 fill a
+# tile, rows of 6152 and of 100 are left to the generic kernels.
+WIDTHS = [(2, 63, 1, 96), (2, 64, 1, 96), (1, 65, 1, 96), (1, 256, 3, 96), (2, 73, 1, 80), (1, 49, 2, 112),
+          (2, 33, 1, 192), (1, 300, 5, 8), (1, 97, 1, 16), (1, 77, 1, 40), (1, 3, 1, 6144), (1, 2, 1, 6152),
+          (1, 5, 3, 100), (2, 49, 1, 128), (1, 17, 1, 256), (1, 200, 1, 64)]
+
+
+@pytest.mark.parametrize("shift", [0, 8])  # payloads 16-byte aligned, or only 8
+@pytest.mark.parametrize("scale_dtype", SCALES)
+@pytest.mark.parametrize("layers,bs,heads,hd", WIDTHS)
+def test_fp8_blocks_of_any_row_width(gpu, layers, bs, heads, hd, scale_dtype, shift):
+    pool = finite_pool(gpu, layers, 5, bs, heads, hd, seed=hd)
+    before = bf16_bits(pool)
+    fp32 = scale_dtype == torch.float32
+    _, offset, stride = ops.entry_layout(ops.pool_layout(pool, scale_dtype), ops.FORMAT_FP8)
+    staging = torch.full((2 * stride + 256,), 0xA5, dtype=torch.uint8, device=gpu)
+    entries = [staging.data_ptr() + shift + i * stride for i in range(2)]
+    ops.save_blocks(pool, [4, 1], entries, ops.FORMAT_FP8, scale_dtype)
+    ops.restore_blocks(pool, [0, 3], entries, ops.FORMAT_FP8, scale_dtype)
+    staged, after = u8(staging), bf16_bits(pool)
+    expect = np.full(staged.shape, 0xA5, dtype=np.uint8)  # gaps and everything past the entries stay as they were
+    for i, (src, dst) in enumerate([(4, 0), (1, 3)]):
+        codes, scales = oracle.save_block_fp8(before, src, fp32)
+        at = shift + i * stride
+        expect[at:at + codes.size] = codes.ravel()
+        expect[at + offset:at + offset + scales.nbytes] = scales.view(np.uint8).ravel()
+        before[:, :, dst] = oracle.dequantize(codes, scales, fp32)
+    assert np.array_equal(staged, expect)
+    assert np.array_equal(after, before)
+
+
+# Token counts whose planes of scales (and, with 3 heads of 40, of codes) are not multiples of 16 bytes.
+@pytest.mark.parametrize("scale_dtype", SCALES)
+@pytest.mark.parametrize("heads,hd,tokens", [(1, 128, 1), (1, 128, 257), (2, 128, 511), (1, 64, 513), (3, 40, 301),
+                                             (1, 256, 255), (3, 96, 512), (1, 112, 299)])
+def test_fp8_tokens_of_any_count_and_width(gpu, heads, hd, tokens, scale_dtype):
+    pool = finite_pool(gpu, 2, 6, 256, heads, hd, seed=tokens)
+    before = bf16_bits(pool)
+    fp32 = scale_dtype == torch.float32
+    table, dest = [4, 1, 2][:-(-tokens // 256)], [0, 5, 3][:-(-tokens // 256)]
+    shape = (2, 2, tokens, heads, hd)
+    payload = torch.empty(shape, dtype=torch.float8_e4m3fn, device=gpu)
+    scale = torch.empty((*shape[:-1], 1), dtype=scale_dtype, device=gpu)
+    ops.gather_tokens_fp8(pool, table, tokens, payload, scale)
+    codes, scales = oracle.quantize(oracle.gather_tokens(before, table, tokens), fp32)
+    assert np.array_equal(u8(payload), codes)
+    assert np.array_equal(u8(scale).ravel(), scales.view(np.uint8).ravel())
+    ops.scatter_tokens_fp8(pool, dest, tokens, payload, scale)
+    oracle.scatter_tokens(before, dest, oracle.dequantize(codes, scales, fp32))
+    assert np.array_equal(bf16_bits(pool), before)
+
+
+@pytest.mark.parametrize("scale_dtype", SCALES)
+@pytest.mark.parametrize("heads,hd", [(3, 96), (1, 80)])
+def test_engine_saves_and_restores_of_other_widths(gpu, heads, hd, scale_dtype):
+    # Saves of 1-2 blocks behind a busy caller are written to the host slots by a capped grid of workgroups.
+    from kvx.engine.cpu_prefix_cache import _CopyEngine
+
+    pool = finite_pool(gpu, 3, 9, 50, heads, hd, seed=7)
+    before = bf16_bits(pool)
+    fp32 = scale_dtype == torch.float32
+    engine = _CopyEngine(pool, ops.pool_layout(pool, scale_dtype), ops.FORMAT_FP8, split=True)
+    try:
+        slab = torch.full((6 * engine.entry_stride,), 0xA5, dtype=torch.uint8, pin_memory=True)
+        staging = [torch.empty(4 * engine.entry_stride, dtype=torch.uint8, device=gpu) for _ in range(2)]
+        engine.add_slab(slab, 6)
+        engine.set_staging(*staging, 4)
+        compute = torch.cuda.current_stream(gpu).cuda_stream
+        for blocks, slots in [([7], [0]), ([2, 5], [1, 2]), ([0, 8, 3], [3, 4, 5])]:
+            ops.sleep(1000, device=gpu)
+            engine.save(blocks, slots, compute)
+        engine.synchronize()
+        for slots, blocks, wait in [([0], [4], True), ([1, 2], [6, 1], False), ([3, 4, 5], [7, 2, 5], True)]:
+            engine.restore(slots, blocks, wait, compute)
+        engine.synchronize()
+        entries = slab.numpy().reshape(6, engine.entry_stride)
+        for slot, (src, dst) in enumerate(zip([7, 2, 5, 0, 8, 3], [4, 6, 1, 7, 2, 5])):
+            codes, scales = oracle.save_block_fp8(before, src, fp32)
+            at = engine.scale_offset
+            assert np.array_equal(entries[slot, :codes.size], codes.ravel()), slot
+            assert np.array_equal(entries[slot, at:at + scales.nbytes], scales.view(np.uint8).ravel()), slot
+            assert np.array_equal(bf16_bits(pool[:, :, dst]), oracle.dequantize(codes, scales, fp32)), slot
+    finally:
+        engine.close()
