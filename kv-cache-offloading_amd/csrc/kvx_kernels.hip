@@ -87,10 +87,11 @@ __device__ __forceinline__ uint32_t load_host32(__amdgpu_buffer_rsrc_t r, int of
 // turn; kChunk < 0 gives each XCD one contiguous eighth of the grid. Measured
 // on the Qwen3-8B block workload: one eighth per XCD (instead of every 8th
 // tile) raised the FP8 kernels from ~5.5 to ~6.2-6.5 TB/s, and no run length
-// beats it for the restore and store_kvcache kernels. The save kernel alone
+// beats it for the restore kernel. The save kernel alone
 // gains ~1% with runs of 1024 tiles, but a restore launched after such a save
 // ran 0.4-0.5% slower, so the save keeps one eighth per XCD too. The BF16
-// copies, with 1 KiB tiles, are fastest in the dispatcher's own order (0).
+// copies, with 1 KiB tiles, and store_kvcache, with one wave per workgroup, are
+// fastest in the dispatcher's own order (0).
 constexpr int kXcds = 8;
 constexpr int kSaveXcdRun = -1;
 constexpr int kCopyXcdRun = 0;
@@ -736,35 +737,50 @@ __global__ __launch_bounds__(kThreads) void raw_copy_generic(uint8_t* __restrict
 // ---------------------------------------------------------------------------
 // store_kvcache (nanovllm/layers/attention.py:10-30)
 
-// Rows of kRow16 uint4: each thread moves one 16-byte piece of a token's K
-// row or V row, kStoreThreads consecutive pieces per workgroup. One access
-// per thread, nontemporal accesses and XCD-contiguous token ranges were the
-// fastest shape on the 16-sequence Qwen3-8B batch (random slots: 4.77 -> 5.29
-// TB/s; contiguous slots: 4.85 -> 5.89 TB/s); several passes per workgroup
-// were slower. Workgroup size and order, as fractions of 8 TB/s (random /
-// paged-block / contiguous slots, two passes agreeing within 0.1 point):
-// 128 threads in eighths 67.2 / 75.1 / 76.4; 256 in eighths 66.6 / 74.3 /
-// 75.4; 64 in eighths 66.9 / 75.0 / 76.2; 64 in dispatch order 66.7 / 75.5 /
-// 77.6; 64 in 64-workgroup runs 65.0 / 71.2 / 75.0.
-constexpr int kStoreThreads = 128;
-constexpr int kStoreXcdRun = -1;
-template <int kRow16>
-__global__ __launch_bounds__(kStoreThreads) void store_kv_vec(const uint4* __restrict__ key, int64_t key_stride16,
-                                                             const uint4* __restrict__ value, int64_t value_stride16,
-                                                             uint4* __restrict__ k_cache, uint4* __restrict__ v_cache,
-                                                             const int32_t* __restrict__ slots, int64_t n,
-                                                             int64_t cache_slots) {
-  // 16-byte piece p of the batch: token p / (2 kRow16), then its K row and its V row.
-  const int64_t p = (int64_t)xcd_tile<kStoreXcdRun>(blockIdx.x, gridDim.x) * kStoreThreads + threadIdx.x;
-  const int64_t t = p / (2 * kRow16);
-  const int within = (int)(p - t * (2 * kRow16));
-  const bool is_v = within >= kRow16;
-  const int col = is_v ? within - kRow16 : within;
+// Rows of row16 uint4: each thread moves one 16-byte piece of a token's K row
+// or V row, workgroups in the dispatcher's own order, so that the pieces in
+// flight are a narrow moving window of the batch. Bound by HBM once a batch
+// is tens of megabytes, by launch and ramp below. Where rows are whole waves
+// (kWaveRow) the token, slot and row are scalar. Measured per call on MI355X
+// (us), each layer's K/V read for the first time: 16,384 Qwen3-8B tokens in
+// paged blocks 24.1 with 64 threads, 25.0 with 128, 25.6 with 256, 26.8 with
+// 1024 (128 threads in one contiguous eighth per XCD 26.0, and 26.4 as the
+// kernel was before, in eighths with vector addressing; random slots 28.7
+// before, 27.3 now); 2,048 tokens 5.15 with 64, 4.89 with 128, 4.85 with 256
+// (5.5 before); 8,192 tokens of 32 heads x 96 34.3 (one workgroup per token and
+// 2-byte pieces before: 51.5). No faster: loading the row before its slot is
+// known. Slower: two pieces per thread, of one row (25.8) or K and V (25.9).
+constexpr int kStoreThreads = 64;
+// Small batches are launched and ramped up faster by larger workgroups. The
+// two sizes cross between 524,288 pieces (1 head x 128, 16,384 tokens: 5.3 us
+// with 256 threads, 5.8 with 64) and 786,432 (32 x 96, 1,024 tokens: 6.9
+// and 6.3).
+constexpr int kStoreSmallThreads = 256;
+constexpr int64_t kStoreSmallPieces = 640 << 10;
+constexpr int64_t kStoreMostPieces = int64_t{1} << 30;  // the kernel counts a launch's pieces in 31 bits
+template <int kBlock, bool kWaveRow>
+__global__ __launch_bounds__(kBlock) void store_kv_vec(const uint4* __restrict__ key, int64_t key_stride16,
+                                                      const uint4* __restrict__ value, int64_t value_stride16,
+                                                      uint4* __restrict__ k_cache, uint4* __restrict__ v_cache,
+                                                      const int32_t* __restrict__ slots, int32_t n, int32_t row16,
+                                                      FastDiv token_of, int64_t cache_slots) {
+  // 16-byte piece p of the batch: token p / (2 row16), then its K row and its V row.
+  const int p = (int)(blockIdx.x * kBlock + threadIdx.x);
+  int t, lane = 0;
+  if (kWaveRow) {  // rows of whole waves: the token, the slot and the row are scalar
+    lane = threadIdx.x % 64;
+    t = __builtin_amdgcn_readfirstlane(token_of(p - lane));
+  } else {
+    t = token_of(p);
+  }
   if (t >= n) return;
+  const int within = p - lane - t * 2 * row16;
+  const bool is_v = within >= row16;
+  const int col = (is_v ? within - row16 : within) + lane;
   const int64_t slot = slots[t];
   if (slot < 0 || slot >= cache_slots) return;
   const uint4 v = load_nt16((is_v ? value : key) + t * (is_v ? value_stride16 : key_stride16) + col);
-  store_nt16((is_v ? v_cache : k_cache) + slot * kRow16 + col, v);
+  store_nt16((is_v ? v_cache : k_cache) + slot * row16 + col, v);
 }
 
 // Any row size / alignment: one workgroup per token, copying granules of T
@@ -1131,23 +1147,24 @@ hipError_t launch_store_kvcache(const void* key, int64_t key_stride, const void*
   const int64_t ks = key_stride * elem_bytes, vs = value_stride * elem_bytes;
   const bool aligned = ((uintptr_t)key | (uintptr_t)value | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0 &&
                        ks % 16 == 0 && vs % 16 == 0 && row_bytes % 16 == 0;
-  auto vec = [&](auto kernel, int row16) {
-    const int64_t grid = (n * 2 * row16 + kStoreThreads - 1) / kStoreThreads;
-    if (grid > INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kStoreThreads), 0, stream, (const uint4*)key, ks / 16,
-                       (const uint4*)value, vs / 16, (uint4*)k_cache, (uint4*)v_cache, slot_mapping, n,
-                       cache_slots);
-    return hipGetLastError();
-  };
-  if (aligned) {
-    switch (row_bytes / 16) {
-      case 8: return vec(store_kv_vec<8>, 8);
-      case 16: return vec(store_kv_vec<16>, 16);
-      case 32: return vec(store_kv_vec<32>, 32);
-      case 64: return vec(store_kv_vec<64>, 64);
-      case 128: return vec(store_kv_vec<128>, 128);
-      default: break;
+  const int64_t row16 = row_bytes / 16;
+  if (aligned && 2 * row16 <= kStoreMostPieces) {
+    // Launches of at most kStoreMostPieces pieces (32 GiB of rows).
+    const int64_t most = kStoreMostPieces / (2 * row16);
+    for (int64_t first = 0; first < n; first += most) {
+      const int64_t count = std::min(most, n - first), pieces = count * 2 * row16;
+      const bool wave_row = row16 % 64 == 0, small = pieces < kStoreSmallPieces;
+      const int threads = small ? kStoreSmallThreads : kStoreThreads;
+      auto kernel = small
+                        ? (wave_row ? store_kv_vec<kStoreSmallThreads, true> : store_kv_vec<kStoreSmallThreads, false>)
+                        : (wave_row ? store_kv_vec<kStoreThreads, true> : store_kv_vec<kStoreThreads, false>);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)((pieces + threads - 1) / threads)), dim3(threads), 0, stream,
+                         (const uint4*)key + first * (ks / 16), ks / 16, (const uint4*)value + first * (vs / 16),
+                         vs / 16, (uint4*)k_cache, (uint4*)v_cache, slot_mapping + first, (int32_t)count,
+                         (int32_t)row16, FastDiv((uint32_t)(2 * row16)), cache_slots);
+      if (const hipError_t err = hipGetLastError(); err != hipSuccess) return err;
     }
+    return hipSuccess;
   }
   // Generic path: granules of the element size when it is 2 or 4 bytes, else bytes.
   const unsigned grid = (unsigned)n;

@@ -103,3 +103,45 @@ def test_engine_saves_and_restores_of_other_widths(gpu, heads, hd, scale_dtype):
             assert np.array_equal(bf16_bits(pool[:, :, dst]), oracle.dequantize(codes, scales, fp32)), slot
     finally:
         engine.close()
+
+
+# Rows of 1 to 512 16-byte pieces: below, at and above a wave, whole waves and not, and one that is not in pieces. The
+# token counts put the batch in the small and in the large launch (from 655,360 pieces on), with ragged last workgroups.
+@pytest.mark.parametrize("heads,hd,tokens", [(1, 8, 1), (1, 8, 70), (3, 8, 333), (5, 64, 513), (63, 8, 65), (1, 512, 3),
+                                             (65, 8, 129), (3, 128, 257), (8, 96, 1000), (32, 128, 33), (6, 100, 50),
+                                             (8, 96, 3415), (8, 128, 2561), (1, 504, 5300)])
+def test_store_kvcache_of_any_row_width(gpu, heads, hd, tokens):
+    g = torch.Generator(device=gpu).manual_seed(tokens)
+    slots_total = tokens + 300
+    bits = torch.randint(-32768, 32768, (2, tokens + slots_total, heads * hd), generator=g, device=gpu).to(torch.int16)
+    key = bits[0, :tokens].view(torch.bfloat16).view(tokens, heads, hd)
+    qkv = torch.zeros((tokens, 3 * heads * hd), dtype=torch.bfloat16, device=gpu)
+    qkv[:, 2 * heads * hd:] = bits[1, :tokens].view(torch.bfloat16)
+    value = qkv[:, 2 * heads * hd:].view(tokens, heads, hd)  # a strided view
+    caches = bits[:, tokens:].clone().view(torch.bfloat16).view(2, 1, slots_total, heads, hd)
+    slots = torch.randperm(slots_total, generator=g, device=gpu)[:tokens].to(torch.int32)
+    slots[torch.rand(tokens, generator=g, device=gpu) < 0.1] = -1
+    slots[-1] = slots_total  # outside the cache
+    expect = [bf16_bits(c).reshape(slots_total, -1) for c in caches]
+    host_slots = slots.cpu().numpy()
+    at = (host_slots >= 0) & (host_slots < slots_total)
+    for cache, rows in zip(expect, (key, value)):
+        cache[host_slots[at]] = bf16_bits(rows).reshape(tokens, -1)[at]
+    ops.store_kvcache(key, value, caches[0], caches[1], slots)
+    for cache, want in zip(caches, expect):
+        assert np.array_equal(bf16_bits(cache).reshape(slots_total, -1), want)
+
+
+def test_store_kvcache_beyond_one_launch(gpu):
+    # More than 2^30 16-byte pieces take several launches. One row expanded over every token; few slots are real.
+    row = torch.randn((1, 8, 128), device=gpu).to(torch.bfloat16)
+    tokens = (1 << 22) + 3
+    slots = torch.full((tokens,), -1, dtype=torch.int32, device=gpu)
+    where = torch.tensor([0, (1 << 22) - 1, 1 << 22, tokens - 1], device=gpu)
+    slots[where] = torch.tensor([5, 0, 7, 3], dtype=torch.int32, device=gpu)
+    caches = torch.zeros((2, 1, 8, 8, 128), dtype=torch.bfloat16, device=gpu)
+    ops.store_kvcache(row.expand(tokens, 8, 128), row.expand(tokens, 8, 128), caches[0], caches[1], slots)
+    for cache in caches:
+        for slot in range(8):
+            want = row[0] if slot in (0, 3, 5, 7) else torch.zeros_like(row[0])
+            assert torch.equal(cache[0, slot], want), slot
