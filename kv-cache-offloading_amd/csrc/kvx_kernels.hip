@@ -84,17 +84,21 @@ __device__ __forceinline__ uint32_t load_host32(__amdgpu_buffer_rsrc_t r, int of
 // Workgroups are dispatched round-robin over the chip's 8 XCDs, each with its
 // own L2. xcd_tile<kChunk> maps workgroup IDs to tiles so that each XCD
 // streams through runs of kChunk consecutive tiles, the XCDs taking runs in
-// turn; kChunk < 0 gives each XCD one contiguous eighth of the grid. Measured
-// on the Qwen3-8B block workload: one eighth per XCD (instead of every 8th
-// tile) raised the FP8 kernels from ~5.5 to ~6.2-6.5 TB/s, and no run length
-// beats it for the restore kernel. The save kernel alone
-// gains ~1% with runs of 1024 tiles, but a restore launched after such a save
-// ran 0.4-0.5% slower, so the save keeps one eighth per XCD too. The BF16
-// copies, with 1 KiB tiles, and store_kvcache, with one wave per workgroup, are
-// fastest in the dispatcher's own order (0).
+// turn; kChunk < 0 gives each XCD one contiguous eighth of the grid, 0 keeps
+// the dispatcher's order. Measured on MI355X (us), Qwen3-8B blocks:
+// - saves, runs of 256 / 1024 / 4096 tiles / eighths / dispatcher's order: 128
+//   blocks 1083 / 1084 / 1091 / 1093 / 1534, 16 blocks 136 / 136 / 140 / 140 /
+//   140, 128 blocks of one KV head 142 / 141 / 145 / 147 / 146;
+// - restores, eighths / runs of 1024 / 256 / 64 / 16 / dispatcher's order: 128
+//   blocks 1143 / 1145 / 1161 / 1230 / 1386 / 1280. Taking the tiles plane by
+//   plane over all entries instead of entry by entry gave 1165 there, 143
+//   against 150 for 16 blocks, but 22.2 against 21.5 for 16 of one KV head;
+// - BF16 copies with 1 KiB tiles, runs of 512 / 128 / 64 / dispatcher's order:
+//   32 Qwen3-0.6B blocks each way 568 / 569 / 587 / 580, 48 Qwen3-8B blocks
+//   1091 / 1087 / 1143 / 1155.
 constexpr int kXcds = 8;
-constexpr int kSaveXcdRun = -1;
-constexpr int kCopyXcdRun = 0;
+constexpr int kSaveXcdRun = 256;
+constexpr int kCopyXcdRun = 512;
 template <int kChunk = -1>
 __device__ __forceinline__ int xcd_tile(int bid, int grid) {
   if (kChunk == 0) return bid;  // the dispatcher's own round-robin order
@@ -313,12 +317,11 @@ struct TileCoord {
 };
 
 __device__ __forceinline__ TileCoord tile_coord_at(const PlaneGeom& g, int tile_rows, int tile) {
-  const int per_entry = g.planes * g.chunks;
   TileCoord t;
-  t.entry = tile / per_entry;
-  const int rem = tile - t.entry * per_entry;
-  t.plane = rem / g.chunks;
-  t.row0 = (rem - t.plane * g.chunks) * tile_rows;
+  const int plane = g.plane_of(tile);  // over all entries
+  t.row0 = (tile - plane * g.chunks) * tile_rows;
+  t.entry = g.entry_of(plane);
+  t.plane = plane - t.entry * g.planes;
   return t;
 }
 
@@ -456,22 +459,6 @@ __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restric
 // 64 x 2048 rows of 96 saved and restored in 201 us against 13,600 (6.05 TB/s),
 // 20,001 tokens of 72 x 2 rows of 128 packed and unpacked in 384 us against
 // 27,000 (5.8 TB/s).
-
-// n / d for 0 <= n < 2^31 and 1 <= d < 2^31 by one multiplication: with
-// 2^l >= d and mul = floor(2^(31 + l) / d) + 1, mul * d exceeds 2^(31 + l) by at
-// most d <= 2^l, so n times that excess stays below 2^(31 + l) and the quotient
-// is exact. mul < 2^33 / 2 fits 32 bits.
-struct FastDiv {
-  uint32_t mul;
-  uint32_t shift;
-  explicit FastDiv(uint32_t d) {
-    uint32_t l = 0;
-    while ((1u << l) < d) ++l;
-    shift = 31 + l;
-    mul = (uint32_t)((uint64_t{1} << shift) / d + 1);
-  }
-  __device__ __forceinline__ int operator()(int n) const { return (int)(((uint64_t)(uint32_t)n * mul) >> shift); }
-};
 
 template <bool kHost>
 __device__ __forceinline__ void store8(void* p, uint2 v) {
@@ -657,8 +644,8 @@ __global__ __launch_bounds__(kThreads) void fp8_restore_generic(uint16_t* __rest
 // RAW (BF16 mode) gather / scatter: byte copies of each block plane.
 
 // Tile shape of the device-side copies: one nontemporal 16-byte piece per
-// thread in 64-thread workgroups (1 KiB tiles), taken in the dispatcher's
-// order. Measured on 128 Qwen3-8B blocks (TB/s, gather / scatter, median of
+// thread in 64-thread workgroups (1 KiB tiles). Measured in the dispatcher's
+// order (xcd_tile has the runs they are taken in now) on 128 Qwen3-8B blocks (TB/s, gather / scatter, median of
 // two passes): 6.71 / 6.62, against 6.28 / 6.31 for 8 KiB tiles of 256
 // threads in 64-tile runs per XCD, 6.59 / 6.58 for 1 KiB tiles in one
 // contiguous eighth per XCD, 6.34 / 6.33 for 2 KiB tiles of 128 threads and
@@ -683,14 +670,11 @@ __global__ __launch_bounds__(kBlock) void raw_copy_kernel(uint8_t* __restrict__ 
                                                          int64_t last_bytes) {
   constexpr int kVecs = kStride ? kStrideCopyVecs : kCopyVecs;
   constexpr int kTileBytes = kBlock * kVecs * 16;
-  const int per_entry = g.planes * g.chunks;
-  const int tiles = kStride ? b.n * per_entry : 1;
+  const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
   for (int t = kStride ? (int)blockIdx.x : 0; t < tiles; t += kStride ? (int)gridDim.x : 1) {
-  const int tile = kStride ? t : xcd_tile<kCopyXcdRun>(blockIdx.x, gridDim.x);
-  const int e = tile / per_entry;
-  const int rem = tile - e * per_entry;
-  const int p = rem / g.chunks;
-  const int64_t off0 = (int64_t)(rem - p * g.chunks) * kTileBytes;
+  const TileCoord tc = tile_coord_at(g, 1, kStride ? t : xcd_tile<kCopyXcdRun>(blockIdx.x, gridDim.x));
+  const int e = tc.entry, p = tc.plane;
+  const int64_t off0 = (int64_t)tc.row0 * kTileBytes;
   const int64_t valid = e == b.n - 1 ? last_bytes : plane_bytes;
   uint8_t* pl = pool + ((int64_t)b.ids[e] * g.block_stride + (int64_t)p * g.plane_stride) * elem_bytes;
   uint8_t* en = reinterpret_cast<uint8_t*>(b.entries[e]) + (int64_t)p * entry_plane_stride;
@@ -918,6 +902,11 @@ __global__ void zero_counters(uint64_t* c) {
 // ---------------------------------------------------------------------------
 // Launchers
 
+static void set_chunks(PlaneGeom& g, int64_t chunks) {
+  g.chunks = (int32_t)chunks;
+  g.plane_of = FastDiv((uint32_t)chunks);
+}
+
 // Geometry of block entries (dense per block); `span` switches FP8 entries to token entries.
 static PlaneGeom make_geom(const kvx_block_layout& l, int tile_rows, int64_t scale_offset,
                            const TokenSpan* span = nullptr) {
@@ -933,7 +922,8 @@ static PlaneGeom make_geom(const kvx_block_layout& l, int tile_rows, int64_t sca
   g.plane_rows = l.plane_rows;
   g.last_rows = span ? span->last_rows : l.plane_rows;
   g.head_dim = l.head_dim;
-  g.chunks = tile_rows > 0 ? (l.plane_rows + tile_rows - 1) / tile_rows : 0;
+  g.entry_of = FastDiv((uint32_t)l.planes);
+  set_chunks(g, tile_rows > 0 ? (l.plane_rows + (int64_t)tile_rows - 1) / tile_rows : 1);
   return g;
 }
 
@@ -955,7 +945,7 @@ static hipError_t launch_fp8_linear(bool save, void* pool, const kvx_block_layou
   if (!save) {
     constexpr int kPieces = kLinearRestoreBlock * kLinearRestoreVecs;
     PlaneGeom g = make_geom(l, 0, scale_offset, span);
-    g.chunks = (int32_t)(((int64_t)l.plane_rows * row_pieces + kPieces - 1) / kPieces);
+    set_chunks(g, ((int64_t)l.plane_rows * row_pieces + kPieces - 1) / kPieces);
     hipLaunchKernelGGL((fp8_restore_linear<kLinearRestoreBlock, kLinearRestoreVecs, kScaleBf16>),
                        dim3((unsigned)(b.n * g.planes * g.chunks)), dim3(kLinearRestoreBlock), 0, stream,
                        (uint16_t*)pool, g, row_of, b);
@@ -1056,7 +1046,7 @@ static hipError_t launch_raw(bool to_entry, void* pool, const kvx_block_layout& 
     auto tiled = [&](int threads, int vecs) {
       const int64_t tile_bytes = (int64_t)threads * vecs * 16;
       PlaneGeom g = make_geom(l, 0, 0);
-      g.chunks = (int32_t)((plane_bytes + tile_bytes - 1) / tile_bytes);
+      set_chunks(g, (plane_bytes + tile_bytes - 1) / tile_bytes);
       return g;
     };
     if (max_grid > 0) {
