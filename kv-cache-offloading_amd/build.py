@@ -1,4 +1,4 @@
-"""Builds libkvx.so (HIP kernels + C ABI) for gfx950 into the kvx package directory.
+"""Builds libkvx.so (HIP kernels + C ABI) for gfx950 and the CPython binding into the kvx package directory.
 
 Run: python kv-cache-offloading_amd/build.py [--arch gfx950] [--verbose]
 """
@@ -14,6 +14,8 @@ HERE = Path(__file__).resolve().parent
 ROOT = HERE.parent
 SOURCES = [HERE / "csrc" / "kvx_kernels.hip", HERE / "csrc" / "kvx_capi.hip"]
 OUTPUT = HERE / "kvx" / "libkvx.so"
+BIND_SOURCE = HERE / "csrc" / "kvx_bind.cpp"
+BIND_OUTPUT = HERE / "kvx" / "_bind.so"
 
 # fp-contract=off keeps every multiply and add separately rounded, as the
 # FP8 codec's bit-exact contract assumes; packed FP32 instructions are
@@ -39,15 +41,37 @@ def build(arch: str = "gfx950", verbose: bool = False) -> Path:
            *map(str, SOURCES), "-o", str(OUTPUT) + ".tmp"]
     if verbose:
         print(" ".join(cmd), flush=True)
-    env = dict(os.environ)
-    result = subprocess.run(cmd, capture_output=True, text=True, env=env)
+    _run(cmd, OUTPUT, verbose)
+    build_bind(verbose)
+    return OUTPUT
+
+
+def build_bind(verbose: bool = False) -> Path:
+    """kvx/_bind.so: host code only, against the installed torch's headers; it calls libkvx by address."""
+    import sysconfig
+
+    import torch
+
+    torch_dir = Path(torch.__file__).parent
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{ROOT / 'include'}",
+           f"-isystem{torch_dir / 'include'}", "-isystem/opt/rocm/include",
+           f"-I{sysconfig.get_paths()['include']}", str(BIND_SOURCE), "-o", str(BIND_OUTPUT) + ".tmp",
+           f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    _run(cmd, BIND_OUTPUT, verbose)
+    return BIND_OUTPUT
+
+
+def _run(cmd: list[str], output: Path, verbose: bool):
+    result = subprocess.run(cmd, capture_output=True, text=True, env=dict(os.environ))
     if result.returncode != 0:
         sys.stderr.write(result.stdout + result.stderr)
-        raise RuntimeError(f"hipcc failed with exit code {result.returncode}")
+        raise RuntimeError(f"{cmd[0]} failed with exit code {result.returncode}")
     if verbose and result.stderr.strip():
         sys.stderr.write(result.stderr)
-    os.replace(str(OUTPUT) + ".tmp", OUTPUT)
-    return OUTPUT
+    os.replace(str(output) + ".tmp", output)
 
 
 def main():

@@ -121,6 +121,27 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_bind = None
+
+
+def bind():
+    """The native operator binding (kvx/_bind.so, csrc/kvx_bind.cpp), calling the loaded libkvx. Raises if not built.
+
+    Each of its functions returns libkvx's status, or None for a call it does not take."""
+    global _bind
+    if _bind is None:
+        handle = lib()
+        try:
+            from kvx import _bind as module
+        except ImportError as e:
+            raise RuntimeError(f"kvx._bind is not built for this torch ({e}): run "
+                               "python kv-cache-offloading_amd/build.py") from e
+        module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
+            handle.kvx_store_kvcache, handle.kvx_save_blocks, handle.kvx_restore_blocks, handle.kvx_entry_layout)))
+        _bind = module
+    return _bind
+
+
 def check(rc: int, what: str = "libkvx"):
     """Raises the Python exception matching a non-zero libkvx return code."""
     if rc == 0:

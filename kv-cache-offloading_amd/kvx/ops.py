@@ -16,6 +16,7 @@ import torch
 
 from kvx import _lib
 from kvx._lib import BlockLayout, check, int32_array, lib, uint64_array
+from kvx._lib import bind as _bind
 
 FORMAT_RAW, FORMAT_FP8 = _lib.FORMAT_RAW, _lib.FORMAT_FP8
 SCALE_DTYPES = {torch.bfloat16: _lib.SCALE_BF16, torch.float32: _lib.SCALE_FP32}
@@ -40,23 +41,8 @@ def _stream(device: torch.device, stream=None) -> int:
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
-# Cache pairs already validated (dtype, contiguity, equal sizes, device), keyed by address, size, row width and
-# dtype: a model binds one pair per layer for the engine's lifetime (model_runner.py:120-126), so each call
-# after the first only repeats the checks that can change from call to call.
-_store_caches: dict[tuple, tuple[int, int]] = {}
-_STORE_CACHE_LIMIT = 4096
-
-
-def _validate_store_caches(k_cache: torch.Tensor, v_cache: torch.Tensor, dtype: torch.dtype, row: int):
-    if not (k_cache.dtype == v_cache.dtype == dtype):
-        raise TypeError("key, value and caches must share one dtype")
-    if not (k_cache.is_contiguous() and v_cache.is_contiguous()) or k_cache.numel() != v_cache.numel():
-        raise ValueError("k_cache and v_cache must be equally sized contiguous slot arrays")
-    device = _require_device(k_cache, v_cache)
-    if len(_store_caches) >= _STORE_CACHE_LIMIT:
-        _store_caches.clear()
-    return k_cache.numel() // row, device.index
-
+# A valid call goes to libkvx straight from the native binding (_lib.bind); one that the binding declines comes back as
+# None and is checked, refused or carried out by the Python below it.
 
 def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                   slot_mapping: torch.Tensor):
@@ -68,11 +54,14 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
     the pool. slot_mapping: int32 [N]; -1 (graph padding) skips a token, and
     so does any slot outside the cache. Capturable in a HIP graph.
 
-    Every call makes the reference's four asserts. A cache pair is checked
-    in full the first time it is seen; later calls with the same pair only
-    check that it is still contiguous, and the inputs' shapes, dtypes and
-    device.
+    Every call makes the reference's four asserts and checks shapes, dtypes
+    and devices.
     """
+    rc = _bind().store(key, value, k_cache, v_cache, slot_mapping)
+    if rc is not None:
+        if rc:
+            check(rc, "store_kvcache")
+        return
     N, num_heads, head_dim = key.shape
     D = num_heads * head_dim
     assert key.stride(-1) == 1 and value.stride(-1) == 1
@@ -80,12 +69,11 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
     assert k_cache.stride(1) == D and v_cache.stride(1) == D
     assert slot_mapping.numel() == N
     dtype = key.dtype
-    k_ptr, v_ptr = k_cache.data_ptr(), v_cache.data_ptr()
-    pair = (k_ptr, v_ptr, k_cache.numel(), v_cache.numel(), D, dtype)
-    known = _store_caches.get(pair)
-    if known is None or not (k_cache.is_contiguous() and v_cache.is_contiguous()):
-        known = _store_caches[pair] = _validate_store_caches(k_cache, v_cache, dtype, D)
-    cache_slots, index = known
+    if not (k_cache.dtype == v_cache.dtype == dtype):
+        raise TypeError("key, value and caches must share one dtype")
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()) or k_cache.numel() != v_cache.numel():
+        raise ValueError("k_cache and v_cache must be equally sized contiguous slot arrays")
+    index = _require_device(k_cache, v_cache).index
     if value.shape != key.shape:
         raise ValueError("key and value shapes differ")
     if value.dtype != dtype:
@@ -97,8 +85,9 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
         raise ValueError("kvx operators need all tensors on one device")
     if N == 0:
         return
-    check(lib().kvx_store_kvcache(key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0), k_ptr, v_ptr,
-                                  slot_mapping.data_ptr(), N, num_heads, head_dim, key.element_size(), cache_slots,
+    check(lib().kvx_store_kvcache(key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0), k_cache.data_ptr(),
+                                  v_cache.data_ptr(), slot_mapping.data_ptr(), N, num_heads, head_dim,
+                                  key.element_size(), k_cache.numel() // D,
                                   torch._C._cuda_getCurrentRawStream(index)), "store_kvcache")
 
 
@@ -145,6 +134,10 @@ def _check_codec(values: torch.Tensor, payload: torch.Tensor, scale: torch.Tenso
 
 
 def _codec(save: bool, values: torch.Tensor, payload: torch.Tensor, scale: torch.Tensor):
+    rc = _bind().codec(save, values, payload, scale)
+    if rc is not None:
+        check(rc, "fp8_quantize" if save else "fp8_dequantize")
+        return
     _check_codec(values, payload, scale)
     device = _require_device(values, payload, scale)
     if values.numel() == 0:
@@ -207,6 +200,11 @@ def entry_layout(layout: BlockLayout, fmt: int) -> tuple[int, int, int]:
 def save_blocks(pool: torch.Tensor, block_ids, entries, fmt: int, scale_dtype: torch.dtype | None = None,
                 stream=None):
     """Queues save (gather [+ FP8 quantise]) of pool blocks into entry addresses."""
+    if stream is None:
+        rc = _bind().blocks(True, pool, block_ids, entries, fmt, scale_dtype)
+        if rc is not None:
+            check(rc, "save_blocks")
+            return
     layout = pool_layout(pool, scale_dtype)
     _, offset, _ = entry_layout(layout, fmt)
     ids, entries = list(block_ids), list(entries)
@@ -220,6 +218,11 @@ def save_blocks(pool: torch.Tensor, block_ids, entries, fmt: int, scale_dtype: t
 def restore_blocks(pool: torch.Tensor, block_ids, entries, fmt: int, scale_dtype: torch.dtype | None = None,
                    stream=None):
     """Queues restore ([FP8 dequantise +] scatter) of entry addresses into pool blocks."""
+    if stream is None:
+        rc = _bind().blocks(False, pool, block_ids, entries, fmt, scale_dtype)
+        if rc is not None:
+            check(rc, "restore_blocks")
+            return
     layout = pool_layout(pool, scale_dtype)
     _, offset, _ = entry_layout(layout, fmt)
     ids, entries = list(block_ids), list(entries)
