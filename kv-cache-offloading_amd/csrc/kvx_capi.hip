@@ -262,11 +262,8 @@ static int token_fp8(bool gather, void* pool, const kvx_block_layout* l, const i
   const uintptr_t payload_bytes = (uintptr_t)(l->planes * num_rows * hd), scale_bytes = (uintptr_t)(l->planes * num_rows * sb);
   if (gather && p0 < s0 + scale_bytes && s0 < p0 + payload_bytes)
     return set_error(KVX_E_INVALID, "payload and scales overlap");
-  // Vector kernels store scales 16 bytes at a time from tile-aligned rows.
-  const bool aligned = p0 % 16 == 0 && s0 % 16 == 0 && (num_rows * hd) % 16 == 0 && (num_rows * sb) % 16 == 0 &&
-                       (R * sb) % 16 == 0;
-  // 8-byte pieces need every plane's payload to start on 8 bytes.
-  const bool pieces = (num_rows * hd) % 8 == 0;
+  // Every plane's payload starts where the first one's alignment allows.
+  const Access planes = num_rows * hd % 16 == 0 ? kVectorAccess : num_rows * hd % 8 == 0 ? kPieceAccess : kAnyAccess;
   TokenSpan span{num_rows * hd, num_rows * sb, R * (sb - hd), (int32_t)R};
   BlockBatch b;
   for (int64_t base = 0; base < nblocks; base += kMaxBatch) {
@@ -278,8 +275,7 @@ static int token_fp8(bool gather, void* pool, const kvx_block_layout* l, const i
     span.last_rows = (int32_t)(base + b.n == nblocks ? num_rows - (nblocks - 1) * R : R);
     // Entry i's scales: scales + (base + i) * R * sb = entries[i] + scale_offset + i * scale_entry_step.
     const int64_t scale_offset = (int64_t)(s0 + (uintptr_t)(base * R * sb)) - (int64_t)(p0 + (uintptr_t)(base * R * hd));
-    Access access = access_of(pool, *l, b.entries, b.n);
-    if (!aligned) access = std::min(access, pieces ? kPieceAccess : kAnyAccess);
+    const Access access = std::min(planes, access_of(pool, *l, b.entries, b.n));
     hipError_t err = launch_token_fp8(gather, pool, *l, b, scale_offset, span, access, stream);
     if (err != hipSuccess) return hip_status(err, gather ? "FP8 token gather launch" : "FP8 token scatter launch");
   }

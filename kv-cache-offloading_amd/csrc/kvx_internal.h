@@ -60,9 +60,11 @@ struct PlaneGeom {
   int32_t plane_rows;
   int32_t last_rows;
   int32_t head_dim;
+  int32_t scales16;      // every plane's scales start on 16 bytes (given 16-byte entries)
   int32_t chunks;        // tiles per plane
   FastDiv plane_of;      // tile -> plane of the batch (/ chunks)
-  FastDiv entry_of;      // plane of the batch -> entry (/ planes)
+  int32_t inner;         // planes, or for token entries the entries of the batch
+  FastDiv outer_of;      // plane of the batch -> entry, or for token entries its plane (/ inner)
 };
 
 // FP8 token entries of one launch (see PlaneGeom).
@@ -83,8 +85,8 @@ int check_layout(const kvx_block_layout* layout, int32_t format);
 // What a pool and its entries' addresses allow. The pool's base and strides
 // are multiples of 16 bytes for the last two, and the entries of 16
 // (kVectorAccess: the tiled kernels) or of 8 (kPieceAccess: FP8 payloads
-// written and read 8 codes at a time, scales one at a time). kAnyAccess runs
-// the element-granular kernels.
+// written and read 8 codes at a time). kAnyAccess runs the element-granular
+// kernels. Scales may start at any element in all of them.
 enum Access { kAnyAccess, kPieceAccess, kVectorAccess };
 
 // Kernel launchers: arguments are validated by the caller.

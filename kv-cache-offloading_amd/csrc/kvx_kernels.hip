@@ -65,6 +65,30 @@ __device__ __forceinline__ void store16(void* p, uint4 v) {
   else store_nt16(p, v);
 }
 
+template <bool kHost>
+__device__ __forceinline__ void store8(void* p, uint2 v) {
+  if (kHost) {
+    u32x2 w = {v.x, v.y};
+    asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" : : "v"(p), "v"(w) : "memory");
+  } else {
+    u32x2 w = {v.x, v.y};
+    __builtin_nontemporal_store(w, reinterpret_cast<u32x2*>(p));
+  }
+}
+
+template <bool kScaleBf16, bool kHost>
+__device__ __forceinline__ void store_scale(uint8_t* scales, int64_t row, uint32_t bits) {
+  if (kScaleBf16) {
+    uint16_t* p = reinterpret_cast<uint16_t*>(scales) + row;
+    if (kHost) asm volatile("global_store_short %0, %1, off sc0 sc1" : : "v"(p), "v"(bits) : "memory");
+    else *p = (uint16_t)bits;
+  } else {
+    uint32_t* p = reinterpret_cast<uint32_t*>(scales) + row;
+    if (kHost) asm volatile("global_store_dword %0, %1, off sc0 sc1" : : "v"(p), "v"(bits) : "memory");
+    else *p = bits;
+  }
+}
+
 // Reads of host memory at system scope (sc0 sc1): never served from a GPU
 // cache line older than the host's or a DMA engine's last write there. Buffer
 // loads through a resource over [base, base + bytes): the compiler tracks them
@@ -82,10 +106,12 @@ __device__ __forceinline__ uint32_t load_host32(__amdgpu_buffer_rsrc_t r, int of
 }
 
 // Workgroups are dispatched round-robin over the chip's 8 XCDs, each with its
-// own L2. xcd_tile<kChunk> maps workgroup IDs to tiles so that each XCD
-// streams through runs of kChunk consecutive tiles, the XCDs taking runs in
-// turn; kChunk < 0 gives each XCD one contiguous eighth of the grid, 0 keeps
-// the dispatcher's order. Measured on MI355X (us), Qwen3-8B blocks:
+// own L2. xcd_tile maps workgroup IDs to tiles: in the dispatcher's order, one
+// contiguous eighth of the grid per XCD, or (orders from 0) so that each XCD
+// streams through runs of 2^order consecutive tiles, the XCDs taking runs in
+// turn. The order is fixed at compile time: read from the geometry, it took
+// 16 blocks of one KV head saved and restored from 42.6 to 43.2 us. Measured on
+// MI355X (us), Qwen3-8B blocks:
 // - saves, runs of 256 / 1024 / 4096 tiles / eighths / dispatcher's order: 128
 //   blocks 1083 / 1084 / 1091 / 1093 / 1534, 16 blocks 136 / 136 / 140 / 140 /
 //   140, 128 blocks of one KV head 142 / 141 / 145 / 147 / 146;
@@ -96,22 +122,31 @@ __device__ __forceinline__ uint32_t load_host32(__amdgpu_buffer_rsrc_t r, int of
 // - BF16 copies with 1 KiB tiles, runs of 512 / 128 / 64 / dispatcher's order:
 //   32 Qwen3-0.6B blocks each way 568 / 569 / 587 / 580, 48 Qwen3-8B blocks
 //   1091 / 1087 / 1143 / 1155.
-constexpr int kXcds = 8;
-constexpr int kSaveXcdRun = 256;
-constexpr int kCopyXcdRun = 512;
-template <int kChunk = -1>
+// Token copies take their tiles plane by plane (TileCoord), which streams
+// through the dense side and stays within one plane of the pool. Gather +
+// scatter, entry by entry in the blocks' orders / plane by plane in those /
+// plane by plane in their own: FP8, 20,001 tokens of 2 KV heads 376 / 350 /
+// 344, 30,001 of one 303 / 271 / 262, 8,001 of 8 571 / 556 / 542; BF16,
+// 30,001 of one 372 / 341 / 333, 8,001 of 8 727 / 711 / 707.
+constexpr int kOrderDispatch = -1;
+constexpr int kOrderEighths = -2;
+template <int kOrder>
 __device__ __forceinline__ int xcd_tile(int bid, int grid) {
-  if (kChunk == 0) return bid;  // the dispatcher's own round-robin order
-  if (kChunk < 0) {
-    const int per = grid / kXcds;
-    if (bid >= per * kXcds) return bid;  // the ragged tail keeps its place
-    return (bid % kXcds) * per + bid / kXcds;
+  if (kOrder == kOrderDispatch) return bid;
+  if (kOrder == kOrderEighths) {
+    const int per = grid / 8;
+    return bid < per * 8 ? (bid % 8) * per + bid / 8 : bid;  // the ragged tail keeps its place
   }
-  const int span = kXcds * kChunk;  // one run for each XCD
-  if (bid >= grid / span * span) return bid;  // likewise
-  const int nth = bid / kXcds;  // this workgroup's place in its XCD's sequence
-  return nth / kChunk * span + (bid % kXcds) * kChunk + nth % kChunk;
+  constexpr int kLog = kOrder < 0 ? 0 : kOrder;
+  const uint32_t nth = (uint32_t)bid >> 3;  // this workgroup's place in its XCD's sequence
+  const uint32_t round = nth >> kLog;       // of one run for each XCD
+  if (round >= (uint32_t)grid >> 3 >> kLog) return bid;  // likewise
+  return (int)((((round << 3) + ((uint32_t)bid & 7)) << kLog) + (nth & ((1u << kLog) - 1)));
 }
+
+constexpr int kSaveOrder = 8, kTokenSaveOrder = 6;
+constexpr int kRestoreOrder = kOrderEighths, kTokenRestoreOrder = kOrderDispatch;
+constexpr int kCopyOrder = 9, kTokenCopyOrder = kOrderDispatch;
 
 // ---------------------------------------------------------------------------
 // Scalar conversions
@@ -316,18 +351,23 @@ struct TileCoord {
   int entry, plane, row0;
 };
 
+// The planes of a batch are taken entry by entry or, for token entries
+// (kTokens), plane by plane over all entries.
+template <bool kTokens>
 __device__ __forceinline__ TileCoord tile_coord_at(const PlaneGeom& g, int tile_rows, int tile) {
   TileCoord t;
-  const int plane = g.plane_of(tile);  // over all entries
+  const int plane = g.plane_of(tile);  // of the batch
   t.row0 = (tile - plane * g.chunks) * tile_rows;
-  t.entry = g.entry_of(plane);
-  t.plane = plane - t.entry * g.planes;
+  const int outer = g.outer_of(plane);
+  const int inner = plane - outer * g.inner;
+  t.entry = kTokens ? inner : outer;
+  t.plane = kTokens ? outer : inner;
   return t;
 }
 
-template <int kChunk>
+template <bool kTokens, int kOrder>
 __device__ __forceinline__ TileCoord tile_coord(const PlaneGeom& g, int tile_rows) {
-  return tile_coord_at(g, tile_rows, xcd_tile<kChunk>(blockIdx.x, gridDim.x));
+  return tile_coord_at<kTokens>(g, tile_rows, xcd_tile<kOrder>(blockIdx.x, gridDim.x));
 }
 
 // Save: one (token, head) row per kLanes lanes, one row per lane group; the
@@ -338,7 +378,7 @@ __device__ __forceinline__ TileCoord tile_coord(const PlaneGeom& g, int tile_row
 // workgroups stride over the tiles, with system-scope stores. Such a launch
 // lasts as long as its writes take to cross the host link; a few workgroups
 // keep the link busy and leave the CUs to other streams' kernels.
-template <int kHd, int kVec, int kBlock, bool kScaleBf16, bool kStride>
+template <int kHd, int kVec, int kBlock, bool kScaleBf16, bool kStride, bool kTokens>
 __global__ __launch_bounds__(kBlock) void fp8_save_kernel(const uint16_t* __restrict__ pool, PlaneGeom g,
                                                          BlockBatch b) {
   using M = RowMap<kHd, kVec>;
@@ -350,7 +390,7 @@ __global__ __launch_bounds__(kBlock) void fp8_save_kernel(const uint16_t* __rest
   const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
   for (int tile = kStride ? (int)blockIdx.x : 0; tile < tiles; tile += kStride ? (int)gridDim.x : 1) {
   if (kStride) __syncthreads();  // the previous tile's stores have read the LDS tile
-  const TileCoord tc = kStride ? tile_coord_at(g, kRows, tile) : tile_coord<kSaveXcdRun>(g, kRows);
+  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, kRows, tile) : tile_coord<kTokens, kTokens ? kTokenSaveOrder : kSaveOrder>(g, kRows);
   const int lane = threadIdx.x % M::kLanes;
   const int rsub = threadIdx.x / M::kLanes;
   const int row = tc.row0 + rsub;
@@ -384,12 +424,11 @@ __global__ __launch_bounds__(kBlock) void fp8_save_kernel(const uint16_t* __rest
   uint8_t* tile_payload = payload + (int64_t)tc.row0 * kHd;
   for (int i = threadIdx.x; i < kRows * kHd / 16; i += kBlock)
     if (full || tc.row0 + i * 16 / kHd < rows) store16<kStride>(tile_payload + i * 16, codes[i]);
-  if (full) {
+  if (full && g.scales16) {
     for (int i = threadIdx.x; i < kRows * kScaleBytes / 16; i += kBlock)
       store16<kStride>(scales + (int64_t)tc.row0 * kScaleBytes + i * 16, scale_tile[i]);
-  } else if (lane == 0 && row < rows) {  // ragged last tile of a plane
-    if (kScaleBf16) reinterpret_cast<uint16_t*>(scales)[row] = (uint16_t)r.bits;
-    else reinterpret_cast<uint32_t*>(scales)[row] = r.bits;
+  } else if (lane == 0 && row < rows) {  // ragged last tile of a plane, or scales at an odd address
+    store_scale<kScaleBf16, kStride>(scales, row, r.bits);
   }
   }
 }
@@ -402,7 +441,7 @@ __global__ __launch_bounds__(kBlock) void fp8_save_kernel(const uint16_t* __rest
 // (one-wave workgroups; 128 and 256 threads gave ~6.48 and ~6.43).
 // kStride: restores read straight from host slots, by a capped grid whose
 // workgroups stride over the tiles (as the striding save instance).
-template <int kHd, int kVec, int kBlock, bool kScaleBf16, bool kStride>
+template <int kHd, int kVec, int kBlock, bool kScaleBf16, bool kStride, bool kTokens>
 __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restrict__ pool, PlaneGeom g,
                                                             BlockBatch b) {
   using M = RowMap<kHd, kVec>;
@@ -412,7 +451,7 @@ __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restric
   const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
   for (int tile = kStride ? (int)blockIdx.x : 0; tile < tiles; tile += kStride ? (int)gridDim.x : 1) {
   if (kStride) __syncthreads();  // the previous tile's codes have been read back
-  const TileCoord tc = kStride ? tile_coord_at(g, kRows, tile) : tile_coord<-1>(g, kRows);
+  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, kRows, tile) : tile_coord<kTokens, kTokens ? kTokenRestoreOrder : kRestoreOrder>(g, kRows);
   const int lane = threadIdx.x % M::kLanes;
   const int rsub = threadIdx.x / M::kLanes;
   const int row = tc.row0 + rsub;
@@ -460,37 +499,13 @@ __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restric
 // 20,001 tokens of 72 x 2 rows of 128 packed and unpacked in 384 us against
 // 27,000 (5.8 TB/s).
 
-template <bool kHost>
-__device__ __forceinline__ void store8(void* p, uint2 v) {
-  if (kHost) {
-    u32x2 w = {v.x, v.y};
-    asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" : : "v"(p), "v"(w) : "memory");
-  } else {
-    u32x2 w = {v.x, v.y};
-    __builtin_nontemporal_store(w, reinterpret_cast<u32x2*>(p));
-  }
-}
-
-template <bool kScaleBf16, bool kHost>
-__device__ __forceinline__ void store_scale(uint8_t* scales, int64_t row, uint32_t bits) {
-  if (kScaleBf16) {
-    uint16_t* p = reinterpret_cast<uint16_t*>(scales) + row;
-    if (kHost) asm volatile("global_store_short %0, %1, off sc0 sc1" : : "v"(p), "v"(bits) : "memory");
-    else *p = (uint16_t)bits;
-  } else {
-    uint32_t* p = reinterpret_cast<uint32_t*>(scales) + row;
-    if (kHost) asm volatile("global_store_dword %0, %1, off sc0 sc1" : : "v"(p), "v"(bits) : "memory");
-    else *p = bits;
-  }
-}
-
 // Save: whole rows per tile, as each row's maximum crosses threads (and waves)
 // through LDS; the scale divisions are then made once per row. kStride as in
 // fp8_save_kernel. Threads x pieces per thread, saving 80 blocks of 64 x 2048
 // rows of 96 / 60 of 64 x 1024 rows of 192 (us): 256 x 3 492 / 371, 256 x 2
 // 512 / 404, 256 x 4 499 / 370, 128 x 4 497 / 374, 64 x 8 508 / 381,
 // 512 x 2 509 / 411, 256 x 1 764.
-template <int kBlock, int kVecs, bool kScaleBf16, bool kStride>
+template <int kBlock, int kVecs, bool kScaleBf16, bool kStride, bool kTokens>
 __global__ __launch_bounds__(kBlock) void fp8_save_linear(const uint16_t* __restrict__ pool, PlaneGeom g,
                                                          int tile_rows, FastDiv row_of, BlockBatch b) {
   constexpr int kPieces = kBlock * kVecs;
@@ -498,7 +513,7 @@ __global__ __launch_bounds__(kBlock) void fp8_save_linear(const uint16_t* __rest
   __shared__ float2 row_params[kPieces];
   const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
   for (int tile = kStride ? (int)blockIdx.x : 0; tile < tiles; tile += kStride ? (int)gridDim.x : 1) {
-    const TileCoord tc = kStride ? tile_coord_at(g, tile_rows, tile) : tile_coord<kSaveXcdRun>(g, tile_rows);
+    const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, tile_rows, tile) : tile_coord<kTokens, kTokens ? kTokenSaveOrder : kSaveOrder>(g, tile_rows);
     const int left = (tc.entry == b.n - 1 ? g.last_rows : g.plane_rows) - tc.row0;
     const int rows = left < tile_rows ? left : tile_rows;  // at most 0 past the end of a partial entry
     const int pieces = rows * (g.head_dim / 8);
@@ -550,10 +565,10 @@ __global__ __launch_bounds__(kBlock) void fp8_save_linear(const uint16_t* __rest
 // plane, wherever its rows begin (80 blocks of 64 x 2048 rows of 96: 505 us,
 // against 524 with whole rows per tile). Threads x pieces: 256 x 2 505,
 // 512 x 2 518, 128 x 4 543, 64 x 4 548, 256 x 3 586, 256 x 1 638.
-template <int kBlock, int kVecs, bool kScaleBf16>
+template <int kBlock, int kVecs, bool kScaleBf16, bool kTokens>
 __global__ __launch_bounds__(kBlock) void fp8_restore_linear(uint16_t* __restrict__ pool, PlaneGeom g, FastDiv row_of,
                                                             BlockBatch b) {
-  const TileCoord tc = tile_coord<-1>(g, kBlock * kVecs);  // row0 counts pieces here
+  const TileCoord tc = tile_coord<kTokens, kTokens ? kTokenRestoreOrder : kRestoreOrder>(g, kBlock * kVecs);  // row0 counts pieces here
   const int pieces = (tc.entry == b.n - 1 ? g.last_rows : g.plane_rows) * (g.head_dim / 8);
   uint16_t* dst = pool + (int64_t)b.ids[tc.entry] * g.block_stride + (int64_t)tc.plane * g.plane_stride;
   const uint8_t* payload =
@@ -663,7 +678,7 @@ constexpr int kStrideCopyVecs = 4;
 // copies last_bytes (a sequence's partial final block in a token gather).
 // kStride: copies to or from host memory by a capped striding grid, as the
 // FP8 kernels' striding instances; writes to host memory use system-scope stores.
-template <bool kToEntry, bool kStride, int kBlock = kStride ? kThreads : kCopyThreads>
+template <bool kToEntry, bool kStride, bool kTokens, int kBlock = kStride ? kThreads : kCopyThreads>
 __global__ __launch_bounds__(kBlock) void raw_copy_kernel(uint8_t* __restrict__ pool, PlaneGeom g,
                                                          BlockBatch b, int64_t plane_bytes,
                                                          int64_t elem_bytes, int64_t entry_plane_stride,
@@ -672,7 +687,7 @@ __global__ __launch_bounds__(kBlock) void raw_copy_kernel(uint8_t* __restrict__ 
   constexpr int kTileBytes = kBlock * kVecs * 16;
   const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
   for (int t = kStride ? (int)blockIdx.x : 0; t < tiles; t += kStride ? (int)gridDim.x : 1) {
-  const TileCoord tc = tile_coord_at(g, 1, kStride ? t : xcd_tile<kCopyXcdRun>(blockIdx.x, gridDim.x));
+  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, 1, t) : tile_coord<kTokens, kTokens ? kTokenCopyOrder : kCopyOrder>(g, 1);
   const int e = tc.entry, p = tc.plane;
   const int64_t off0 = (int64_t)tc.row0 * kTileBytes;
   const int64_t valid = e == b.n - 1 ? last_bytes : plane_bytes;
@@ -908,8 +923,8 @@ static void set_chunks(PlaneGeom& g, int64_t chunks) {
 }
 
 // Geometry of block entries (dense per block); `span` switches FP8 entries to token entries.
-static PlaneGeom make_geom(const kvx_block_layout& l, int tile_rows, int64_t scale_offset,
-                           const TokenSpan* span = nullptr) {
+static PlaneGeom make_geom(const kvx_block_layout& l, const BlockBatch& b, bool tokens, int tile_rows,
+                           int64_t scale_offset, const TokenSpan* span = nullptr) {
   PlaneGeom g;
   g.plane_stride = l.plane_stride;
   g.block_stride = l.block_stride;
@@ -922,7 +937,9 @@ static PlaneGeom make_geom(const kvx_block_layout& l, int tile_rows, int64_t sca
   g.plane_rows = l.plane_rows;
   g.last_rows = span ? span->last_rows : l.plane_rows;
   g.head_dim = l.head_dim;
-  g.entry_of = FastDiv((uint32_t)l.planes);
+  g.scales16 = (scale_offset | g.scale_plane_stride | g.scale_entry_step) % 16 == 0;
+  g.inner = tokens ? b.n : l.planes;
+  g.outer_of = FastDiv((uint32_t)g.inner);
   set_chunks(g, tile_rows > 0 ? (l.plane_rows + (int64_t)tile_rows - 1) / tile_rows : 1);
   return g;
 }
@@ -936,7 +953,7 @@ constexpr int kLinearRestoreBlock = 256;
 constexpr int kLinearRestoreVecs = 2;
 constexpr int kLinearMaxPieces = kLinearSaveBlock * kLinearSaveVecs;  // a row must fit a save tile
 
-template <bool kScaleBf16>
+template <bool kScaleBf16, bool kTokens>
 static hipError_t launch_fp8_linear(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
                                     int64_t scale_offset, int32_t max_grid, hipStream_t stream,
                                     const TokenSpan* span) {
@@ -944,9 +961,9 @@ static hipError_t launch_fp8_linear(bool save, void* pool, const kvx_block_layou
   const FastDiv row_of((uint32_t)row_pieces);
   if (!save) {
     constexpr int kPieces = kLinearRestoreBlock * kLinearRestoreVecs;
-    PlaneGeom g = make_geom(l, 0, scale_offset, span);
+    PlaneGeom g = make_geom(l, b, kTokens, 0, scale_offset, span);
     set_chunks(g, ((int64_t)l.plane_rows * row_pieces + kPieces - 1) / kPieces);
-    hipLaunchKernelGGL((fp8_restore_linear<kLinearRestoreBlock, kLinearRestoreVecs, kScaleBf16>),
+    hipLaunchKernelGGL((fp8_restore_linear<kLinearRestoreBlock, kLinearRestoreVecs, kScaleBf16, kTokens>),
                        dim3((unsigned)(b.n * g.planes * g.chunks)), dim3(kLinearRestoreBlock), 0, stream,
                        (uint16_t*)pool, g, row_of, b);
     return hipGetLastError();
@@ -955,19 +972,19 @@ static hipError_t launch_fp8_linear(bool save, void* pool, const kvx_block_layou
   const int32_t most = kLinearSaveBlock * kLinearSaveVecs / row_pieces;
   const int32_t lines = 128 / std::min(128, l.head_dim & -l.head_dim);
   const int32_t rows = most >= lines ? most / lines * lines : most;
-  const PlaneGeom g = make_geom(l, rows, scale_offset, span);
+  const PlaneGeom g = make_geom(l, b, kTokens, rows, scale_offset, span);
   const unsigned grid = (unsigned)(b.n * g.planes * g.chunks);
   if (max_grid > 0)
-    hipLaunchKernelGGL((fp8_save_linear<kLinearSaveBlock, kLinearSaveVecs, kScaleBf16, true>),
+    hipLaunchKernelGGL((fp8_save_linear<kLinearSaveBlock, kLinearSaveVecs, kScaleBf16, true, kTokens>),
                        dim3(std::min((unsigned)max_grid, grid)), dim3(kLinearSaveBlock), 0, stream,
                        (const uint16_t*)pool, g, rows, row_of, b);
   else
-    hipLaunchKernelGGL((fp8_save_linear<kLinearSaveBlock, kLinearSaveVecs, kScaleBf16, false>), dim3(grid),
+    hipLaunchKernelGGL((fp8_save_linear<kLinearSaveBlock, kLinearSaveVecs, kScaleBf16, false, kTokens>), dim3(grid),
                        dim3(kLinearSaveBlock), 0, stream, (const uint16_t*)pool, g, rows, row_of, b);
   return hipGetLastError();
 }
 
-template <bool kScaleBf16>
+template <bool kScaleBf16, bool kTokens>
 static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
                              int64_t scale_offset, Access access, int32_t max_grid, hipStream_t stream,
                              const TokenSpan* span = nullptr) {
@@ -980,7 +997,7 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
   constexpr int kRestoreStrideBlock = 256;
   auto run = [&](auto save_k, auto save_stride_k, auto restore_k, auto restore_stride_k, int lanes) -> hipError_t {
     const int block = save ? kSaveBlock : kRestoreBlock;
-    PlaneGeom g = make_geom(l, block / lanes, scale_offset, span);
+    PlaneGeom g = make_geom(l, b, kTokens, block / lanes, scale_offset, span);
     const unsigned grid = (unsigned)(b.n * g.planes * g.chunks);
     if (save && max_grid > 0 && (unsigned)max_grid < grid) {
       hipLaunchKernelGGL(save_stride_k, dim3((unsigned)max_grid), dim3(kSaveBlock), 0, stream, (const uint16_t*)pool,
@@ -988,7 +1005,7 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
     } else if (save) {
       hipLaunchKernelGGL(save_k, dim3(grid), dim3(kSaveBlock), 0, stream, (const uint16_t*)pool, g, b);
     } else if (max_grid > 0) {
-      PlaneGeom gs = make_geom(l, kRestoreStrideBlock / lanes, scale_offset, span);
+      PlaneGeom gs = make_geom(l, b, kTokens, kRestoreStrideBlock / lanes, scale_offset, span);
       const unsigned tiles = (unsigned)(b.n * gs.planes * gs.chunks);
       hipLaunchKernelGGL(restore_stride_k, dim3((unsigned)max_grid < tiles ? (unsigned)max_grid : tiles), dim3(kRestoreStrideBlock), 0,
                          stream, (uint16_t*)pool, gs, b);
@@ -999,20 +1016,20 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
   };
   switch (access == kVectorAccess ? l.head_dim : 0) {
     case 64:
-      return run(fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, false>,
-                 fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, true>,
-                 fp8_restore_kernel<64, 1, kRestoreBlock, kScaleBf16, false>,
-                 fp8_restore_kernel<64, 1, kRestoreStrideBlock, kScaleBf16, true>, RowMap<64, 1>::kLanes);
+      return run(fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, false, kTokens>,
+                 fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, true, kTokens>,
+                 fp8_restore_kernel<64, 1, kRestoreBlock, kScaleBf16, false, kTokens>,
+                 fp8_restore_kernel<64, 1, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<64, 1>::kLanes);
     case 128:
-      return run(fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, false>,
-                 fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, true>,
-                 fp8_restore_kernel<128, 2, kRestoreBlock, kScaleBf16, false>,
-                 fp8_restore_kernel<128, 2, kRestoreStrideBlock, kScaleBf16, true>, RowMap<128, 2>::kLanes);
+      return run(fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, false, kTokens>,
+                 fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, true, kTokens>,
+                 fp8_restore_kernel<128, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
+                 fp8_restore_kernel<128, 2, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<128, 2>::kLanes);
     case 256:
-      return run(fp8_save_kernel<256, 2, kSaveBlock, kScaleBf16, false>,
-                 fp8_save_kernel<256, 2, kSaveBlock, kScaleBf16, true>,
-                 fp8_restore_kernel<256, 2, kRestoreBlock, kScaleBf16, false>,
-                 fp8_restore_kernel<256, 2, kRestoreStrideBlock, kScaleBf16, true>, RowMap<256, 2>::kLanes);
+      return run(fp8_save_kernel<256, 2, kSaveBlock, kScaleBf16, false, kTokens>,
+                 fp8_save_kernel<256, 2, kSaveBlock, kScaleBf16, true, kTokens>,
+                 fp8_restore_kernel<256, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
+                 fp8_restore_kernel<256, 2, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<256, 2>::kLanes);
     default: {
       // Rows of other widths, and head_dim 64, 128 or 256 whose payloads or
       // scales are not 16-byte aligned (a handoff of a token count that is not
@@ -1020,8 +1037,8 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
       // tuned widths too but save 128 Qwen3-8B blocks in 1,160 us against
       // fp8_save_kernel's 1,123 and restore them in 1,161 against 1,147.
       if (access != kAnyAccess && l.head_dim % 8 == 0 && l.head_dim / 8 <= kLinearMaxPieces)
-        return launch_fp8_linear<kScaleBf16>(save, pool, l, b, scale_offset, max_grid, stream, span);
-      PlaneGeom g = make_geom(l, 0, scale_offset, span);
+        return launch_fp8_linear<kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
+      PlaneGeom g = make_geom(l, b, kTokens, 0, scale_offset, span);
       const unsigned grid = generic_grid((int64_t)b.n * l.planes * l.plane_rows);
       if (save)
         hipLaunchKernelGGL(fp8_save_generic<kScaleBf16>, dim3(grid), dim3(kThreads), 0, stream,
@@ -1034,6 +1051,7 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
   }
 }
 
+template <bool kTokens>
 static hipError_t launch_raw(bool to_entry, void* pool, const kvx_block_layout& l, const BlockBatch& b,
                              Access access, int64_t entry_plane_stride, int64_t last_bytes, int32_t max_grid,
                              hipStream_t stream) {
@@ -1045,7 +1063,7 @@ static hipError_t launch_raw(bool to_entry, void* pool, const kvx_block_layout& 
   if (vec) {
     auto tiled = [&](int threads, int vecs) {
       const int64_t tile_bytes = (int64_t)threads * vecs * 16;
-      PlaneGeom g = make_geom(l, 0, 0);
+      PlaneGeom g = make_geom(l, b, kTokens, 0, 0);
       set_chunks(g, (plane_bytes + tile_bytes - 1) / tile_bytes);
       return g;
     };
@@ -1053,10 +1071,10 @@ static hipError_t launch_raw(bool to_entry, void* pool, const kvx_block_layout& 
       const PlaneGeom g = tiled(kThreads, kStrideCopyVecs);
       if ((unsigned)max_grid < (unsigned)(b.n * g.planes * g.chunks)) {
         if (to_entry)
-          hipLaunchKernelGGL((raw_copy_kernel<true, true>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
+          hipLaunchKernelGGL((raw_copy_kernel<true, true, kTokens>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
                              (uint8_t*)pool, g, b, plane_bytes, es, entry_plane_stride, last_bytes);
         else
-          hipLaunchKernelGGL((raw_copy_kernel<false, true>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
+          hipLaunchKernelGGL((raw_copy_kernel<false, true, kTokens>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
                              (uint8_t*)pool, g, b, plane_bytes, es, entry_plane_stride, last_bytes);
         return hipGetLastError();
       }
@@ -1064,13 +1082,13 @@ static hipError_t launch_raw(bool to_entry, void* pool, const kvx_block_layout& 
     const PlaneGeom g = tiled(kCopyThreads, kCopyVecs);
     const unsigned grid = (unsigned)(b.n * g.planes * g.chunks);
     if (to_entry)
-      hipLaunchKernelGGL((raw_copy_kernel<true, false>), dim3(grid), dim3(kCopyThreads), 0, stream, (uint8_t*)pool, g,
+      hipLaunchKernelGGL((raw_copy_kernel<true, false, kTokens>), dim3(grid), dim3(kCopyThreads), 0, stream, (uint8_t*)pool, g,
                          b, plane_bytes, es, entry_plane_stride, last_bytes);
     else
-      hipLaunchKernelGGL((raw_copy_kernel<false, false>), dim3(grid), dim3(kCopyThreads), 0, stream, (uint8_t*)pool,
+      hipLaunchKernelGGL((raw_copy_kernel<false, false, kTokens>), dim3(grid), dim3(kCopyThreads), 0, stream, (uint8_t*)pool,
                          g, b, plane_bytes, es, entry_plane_stride, last_bytes);
   } else {
-    PlaneGeom g = make_geom(l, 0, 0);
+    PlaneGeom g = make_geom(l, b, kTokens, 0, 0);
     const unsigned grid = generic_grid((int64_t)b.n * l.planes * (plane_bytes / 2));
     if (to_entry)
       hipLaunchKernelGGL(raw_copy_generic<true>, dim3(grid), dim3(kThreads), 0, stream, (uint8_t*)pool, g, b,
@@ -1085,15 +1103,15 @@ static hipError_t launch_raw(bool to_entry, void* pool, const kvx_block_layout& 
 hipError_t launch_token_copy(bool gather, void* pool, const kvx_block_layout& l, const BlockBatch& b,
                              Access access, int64_t dense_plane_stride, int64_t last_bytes, hipStream_t stream) {
   if (b.n <= 0) return hipSuccess;
-  return launch_raw(gather, pool, l, b, access, dense_plane_stride, last_bytes, 0, stream);
+  return launch_raw<true>(gather, pool, l, b, access, dense_plane_stride, last_bytes, 0, stream);
 }
 
 hipError_t launch_token_fp8(bool gather, void* pool, const kvx_block_layout& l, const BlockBatch& b,
                             int64_t scale_offset, const TokenSpan& span, Access access, hipStream_t stream) {
   if (b.n <= 0) return hipSuccess;
   return l.scale_dtype == KVX_SCALE_BF16
-             ? launch_fp8<true>(gather, pool, l, b, scale_offset, access, 0, stream, &span)
-             : launch_fp8<false>(gather, pool, l, b, scale_offset, access, 0, stream, &span);
+             ? launch_fp8<true, true>(gather, pool, l, b, scale_offset, access, 0, stream, &span)
+             : launch_fp8<false, true>(gather, pool, l, b, scale_offset, access, 0, stream, &span);
 }
 
 Access access_of(const void* pool, const kvx_block_layout& l, const uint64_t* entries, int32_t n) {
@@ -1108,10 +1126,10 @@ hipError_t launch_save(const void* pool, const kvx_block_layout& l, int32_t form
                        int64_t scale_offset, Access access, int32_t max_grid, hipStream_t stream) {
   if (b.n <= 0) return hipSuccess;
   void* p = const_cast<void*>(pool);
-  if (format == KVX_FORMAT_RAW) return launch_raw(true, p, l, b, access, -1, -1, max_grid, stream);
+  if (format == KVX_FORMAT_RAW) return launch_raw<false>(true, p, l, b, access, -1, -1, max_grid, stream);
   return l.scale_dtype == KVX_SCALE_BF16
-             ? launch_fp8<true>(true, p, l, b, scale_offset, access, max_grid, stream)
-             : launch_fp8<false>(true, p, l, b, scale_offset, access, max_grid, stream);
+             ? launch_fp8<true, false>(true, p, l, b, scale_offset, access, max_grid, stream)
+             : launch_fp8<false, false>(true, p, l, b, scale_offset, access, max_grid, stream);
 }
 
 bool striding_restore_supported(const kvx_block_layout& l, int32_t format, Access access) {
@@ -1123,10 +1141,10 @@ bool striding_restore_supported(const kvx_block_layout& l, int32_t format, Acces
 hipError_t launch_restore(void* pool, const kvx_block_layout& l, int32_t format, const BlockBatch& b,
                           int64_t scale_offset, Access access, int32_t max_grid, hipStream_t stream) {
   if (b.n <= 0) return hipSuccess;
-  if (format == KVX_FORMAT_RAW) return launch_raw(false, pool, l, b, access, -1, -1, max_grid, stream);
+  if (format == KVX_FORMAT_RAW) return launch_raw<false>(false, pool, l, b, access, -1, -1, max_grid, stream);
   return l.scale_dtype == KVX_SCALE_BF16
-             ? launch_fp8<true>(false, pool, l, b, scale_offset, access, max_grid, stream)
-             : launch_fp8<false>(false, pool, l, b, scale_offset, access, max_grid, stream);
+             ? launch_fp8<true, false>(false, pool, l, b, scale_offset, access, max_grid, stream)
+             : launch_fp8<false, false>(false, pool, l, b, scale_offset, access, max_grid, stream);
 }
 
 hipError_t launch_store_kvcache(const void* key, int64_t key_stride, const void* value, int64_t value_stride,
