@@ -471,9 +471,13 @@ __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restric
     for (int i = threadIdx.x; i < kPieces; i += kBlock) codes[i] = load_host16(rc, i * 16);
     if (row < rows) s = scale_value_host(host_rsrc(scales, (int64_t)rows * (kScaleBf16 ? 2 : 4)), row, kScaleBf16);
   } else {
+    // The scales' place before or after the codes' loads is measured: fp32 first
+    // (16 blocks 147.0 us, after 148.2; 30 blocks of 4 x 256 293 and 299.5),
+    // bf16 after (64 blocks 582, first 596; 16 blocks of one KV head 22.0, 22.8).
+    if (!kScaleBf16 && row < rows) s = scale_value(scales, row, false);
     for (int i = threadIdx.x; i < kPieces; i += kBlock)
       codes[i] = tc.row0 + i * 16 / kHd < rows ? load_nt16(tile_codes + i * 16) : make_uint4(0, 0, 0, 0);
-    if (row < rows) s = scale_value(scales, row, kScaleBf16);
+    if (kScaleBf16 && row < rows) s = scale_value(scales, row, true);
   }
   __syncthreads();
   if (row < rows) {
@@ -495,9 +499,8 @@ __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restric
 // bf16 and 512 bytes of codes per instruction, in whole 128-byte lines. Bound
 // by HBM. Measured on MI355X against the one-thread-per-row kernels that ran
 // before (2-byte loads and 1-byte stores a row apart, 0.09 TB/s): 16 blocks of
-// 64 x 2048 rows of 96 saved and restored in 201 us against 13,600 (6.05 TB/s),
-// 20,001 tokens of 72 x 2 rows of 128 packed and unpacked in 384 us against
-// 27,000 (5.8 TB/s).
+// 64 x 2048 rows of 96 saved and restored in 198 us against 13,400 (6.1 TB/s),
+// 9,001 tokens of 64 x 4 such rows packed and unpacked in 215 us against 14,900.
 
 // Save: whole rows per tile, as each row's maximum crosses threads (and waves)
 // through LDS; the scale divisions are then made once per row. kStride as in
@@ -1014,11 +1017,15 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
     }
     return hipGetLastError();
   };
-  switch (access == kVectorAccess ? l.head_dim : 0) {
+  // Rows of 64 fill half of a restore wave's code loads: only their striding
+  // kernels are used. The linear kernels restore 100 blocks of 64 x 1024 such
+  // rows in 210 us (245 here) and save them in 201 us (242).
+  const bool tuned = access == kVectorAccess && (l.head_dim != 64 || max_grid > 0);
+  switch (tuned ? l.head_dim : 0) {
     case 64:
-      return run(fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, false, kTokens>,
+      return run(fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, true, kTokens>,
                  fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, true, kTokens>,
-                 fp8_restore_kernel<64, 1, kRestoreBlock, kScaleBf16, false, kTokens>,
+                 fp8_restore_kernel<64, 1, kRestoreStrideBlock, kScaleBf16, true, kTokens>,
                  fp8_restore_kernel<64, 1, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<64, 1>::kLanes);
     case 128:
       return run(fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, false, kTokens>,
@@ -1031,11 +1038,10 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
                  fp8_restore_kernel<256, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
                  fp8_restore_kernel<256, 2, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<256, 2>::kLanes);
     default: {
-      // Rows of other widths, and head_dim 64, 128 or 256 whose payloads or
-      // scales are not 16-byte aligned (a handoff of a token count that is not
-      // a multiple of 16 bytes of scales): the linear kernels, which take the
-      // tuned widths too but save 128 Qwen3-8B blocks in 1,160 us against
-      // fp8_save_kernel's 1,123 and restore them in 1,161 against 1,147.
+      // Other widths, and payloads on 8 bytes only: the linear kernels. They
+      // take rows of 128 and 256 too, but save 128 Qwen3-8B blocks in 1,131 us
+      // against fp8_save_kernel's 1,085 and restore them in 1,158 against
+      // fp8_restore_kernel's 1,143.
       if (access != kAnyAccess && l.head_dim % 8 == 0 && l.head_dim / 8 <= kLinearMaxPieces)
         return launch_fp8_linear<kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
       PlaneGeom g = make_geom(l, b, kTokens, 0, scale_offset, span);
