@@ -147,6 +147,11 @@ __device__ __forceinline__ int xcd_tile(int bid, int grid) {
 constexpr int kSaveOrder = 8, kTokenSaveOrder = 6;
 constexpr int kRestoreOrder = kOrderEighths, kTokenRestoreOrder = kOrderDispatch;
 constexpr int kCopyOrder = 9, kTokenCopyOrder = kOrderDispatch;
+// Smaller copies leave no whole number of run rounds and keep the dispatcher's
+// order: 147,456 tiles (4 Qwen3-8B blocks each way) 98.4 us, 99.2 in runs of
+// 512; 294,912 tiles 184.0 and 181.9; 64 blocks of 72 x 1024 rows of 128
+// (1.18 M tiles) 936 and 757.
+constexpr unsigned kCopyRunTiles = 192 << 10;
 
 // ---------------------------------------------------------------------------
 // Scalar conversions
@@ -681,7 +686,7 @@ constexpr int kStrideCopyVecs = 4;
 // copies last_bytes (a sequence's partial final block in a token gather).
 // kStride: copies to or from host memory by a capped striding grid, as the
 // FP8 kernels' striding instances; writes to host memory use system-scope stores.
-template <bool kToEntry, bool kStride, bool kTokens, int kBlock = kStride ? kThreads : kCopyThreads>
+template <bool kToEntry, bool kStride, bool kTokens, int kOrder, int kBlock = kStride ? kThreads : kCopyThreads>
 __global__ __launch_bounds__(kBlock) void raw_copy_kernel(uint8_t* __restrict__ pool, PlaneGeom g,
                                                          BlockBatch b, int64_t plane_bytes,
                                                          int64_t elem_bytes, int64_t entry_plane_stride,
@@ -690,7 +695,7 @@ __global__ __launch_bounds__(kBlock) void raw_copy_kernel(uint8_t* __restrict__ 
   constexpr int kTileBytes = kBlock * kVecs * 16;
   const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
   for (int t = kStride ? (int)blockIdx.x : 0; t < tiles; t += kStride ? (int)gridDim.x : 1) {
-  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, 1, t) : tile_coord<kTokens, kTokens ? kTokenCopyOrder : kCopyOrder>(g, 1);
+  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, 1, t) : tile_coord<kTokens, kOrder>(g, 1);
   const int e = tc.entry, p = tc.plane;
   const int64_t off0 = (int64_t)tc.row0 * kTileBytes;
   const int64_t valid = e == b.n - 1 ? last_bytes : plane_bytes;
@@ -1077,22 +1082,23 @@ static hipError_t launch_raw(bool to_entry, void* pool, const kvx_block_layout& 
       const PlaneGeom g = tiled(kThreads, kStrideCopyVecs);
       if ((unsigned)max_grid < (unsigned)(b.n * g.planes * g.chunks)) {
         if (to_entry)
-          hipLaunchKernelGGL((raw_copy_kernel<true, true, kTokens>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
+          hipLaunchKernelGGL((raw_copy_kernel<true, true, kTokens, kOrderDispatch>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
                              (uint8_t*)pool, g, b, plane_bytes, es, entry_plane_stride, last_bytes);
         else
-          hipLaunchKernelGGL((raw_copy_kernel<false, true, kTokens>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
+          hipLaunchKernelGGL((raw_copy_kernel<false, true, kTokens, kOrderDispatch>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
                              (uint8_t*)pool, g, b, plane_bytes, es, entry_plane_stride, last_bytes);
         return hipGetLastError();
       }
     }
     const PlaneGeom g = tiled(kCopyThreads, kCopyVecs);
     const unsigned grid = (unsigned)(b.n * g.planes * g.chunks);
-    if (to_entry)
-      hipLaunchKernelGGL((raw_copy_kernel<true, false, kTokens>), dim3(grid), dim3(kCopyThreads), 0, stream, (uint8_t*)pool, g,
-                         b, plane_bytes, es, entry_plane_stride, last_bytes);
-    else
-      hipLaunchKernelGGL((raw_copy_kernel<false, false, kTokens>), dim3(grid), dim3(kCopyThreads), 0, stream, (uint8_t*)pool,
-                         g, b, plane_bytes, es, entry_plane_stride, last_bytes);
+    constexpr int kRuns = kTokens ? kTokenCopyOrder : kCopyOrder;
+    auto kernel = grid < kCopyRunTiles ? (to_entry ? raw_copy_kernel<true, false, kTokens, kOrderDispatch>
+                                                   : raw_copy_kernel<false, false, kTokens, kOrderDispatch>)
+                                       : (to_entry ? raw_copy_kernel<true, false, kTokens, kRuns>
+                                                   : raw_copy_kernel<false, false, kTokens, kRuns>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kCopyThreads), 0, stream, (uint8_t*)pool, g, b, plane_bytes, es,
+                       entry_plane_stride, last_bytes);
   } else {
     PlaneGeom g = make_geom(l, b, kTokens, 0, 0);
     const unsigned grid = generic_grid((int64_t)b.n * l.planes * (plane_bytes / 2));
