@@ -960,36 +960,71 @@ constexpr int kLinearSaveVecs = 3;
 constexpr int kLinearRestoreBlock = 256;
 constexpr int kLinearRestoreVecs = 2;
 constexpr int kLinearMaxPieces = kLinearSaveBlock * kLinearSaveVecs;  // a row must fit a save tile
+// Small planes and small launches take one-wave workgroups with fewer pieces
+// per thread. A launch of many planes is bound by dispatch, which starts four
+// of these for one of 256 threads, and a small launch by the latency of one
+// workgroup, its barriers and its memory passes. Measured on MI355X (us, in a
+// captured graph), workgroups of 256 threads / of one wave:
+// - 16,384 planes of 8 rows of 64: save 15.3 / 7.5, restore 13.4 / 6.9; of one
+//   row of 96: 14.9 / 6.2 and 13.1 / 5.6;
+// - planes of 192 pieces (4,608 of 16 rows of 96): save 7.3 / 6.9, restore 6.65
+//   / 6.4; of 256 pieces (4,096 of 32 rows of 64): 7.3 / 5.9 but 6.7 / 6.8;
+// - one plane of 24,500 rows of 64 (196,000 pieces): save 3.7 / 3.4, restore
+//   3.2 / 3.15; of 32,768 (262,144): 3.95 / 3.55 but 3.45 / 3.6.
+// Token copies keep the larger ones: 17 tokens of 72 planes of one head of 64
+// gathered in 2.3 us, 2.7 with one wave.
+constexpr int kLinearSmallBlock = 64;
+constexpr int kLinearSmallSaveVecs = 2;
+constexpr int kLinearSmallRestoreVecs = 1;
+constexpr int64_t kLinearSmallPlane = 192;
+constexpr int64_t kLinearSmallTotal = 192 << 10;
+// Saves of rows of 64 up to here are latency-bound and stay with the tiled
+// kernel, whose row maxima need no barrier: 2,048 rows 2.4 us (2.7 with the
+// linear one), 4,096 2.75 (2.9), 8,200 3.0 (3.0).
+constexpr int64_t kTiledSave64Rows = 8192;
 
-template <bool kScaleBf16, bool kTokens>
-static hipError_t launch_fp8_linear(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
-                                    int64_t scale_offset, int32_t max_grid, hipStream_t stream,
-                                    const TokenSpan* span) {
+template <int kSaveBlock, int kSaveVecs, int kRestoreBlock, int kRestoreVecs, bool kScaleBf16, bool kTokens>
+static hipError_t launch_fp8_linear_as(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
+                                       int64_t scale_offset, int32_t max_grid, hipStream_t stream,
+                                       const TokenSpan* span) {
   const int32_t row_pieces = l.head_dim / 8;
   const FastDiv row_of((uint32_t)row_pieces);
   if (!save) {
-    constexpr int kPieces = kLinearRestoreBlock * kLinearRestoreVecs;
+    constexpr int kPieces = kRestoreBlock * kRestoreVecs;
     PlaneGeom g = make_geom(l, b, kTokens, 0, scale_offset, span);
     set_chunks(g, ((int64_t)l.plane_rows * row_pieces + kPieces - 1) / kPieces);
-    hipLaunchKernelGGL((fp8_restore_linear<kLinearRestoreBlock, kLinearRestoreVecs, kScaleBf16, kTokens>),
-                       dim3((unsigned)(b.n * g.planes * g.chunks)), dim3(kLinearRestoreBlock), 0, stream,
+    hipLaunchKernelGGL((fp8_restore_linear<kRestoreBlock, kRestoreVecs, kScaleBf16, kTokens>),
+                       dim3((unsigned)(b.n * g.planes * g.chunks)), dim3(kRestoreBlock), 0, stream,
                        (uint16_t*)pool, g, row_of, b);
     return hipGetLastError();
   }
   // As many rows as fit, in whole 128-byte lines of codes (and of bf16) if any such number fits.
-  const int32_t most = kLinearSaveBlock * kLinearSaveVecs / row_pieces;
+  const int32_t most = kSaveBlock * kSaveVecs / row_pieces;
   const int32_t lines = 128 / std::min(128, l.head_dim & -l.head_dim);
   const int32_t rows = most >= lines ? most / lines * lines : most;
   const PlaneGeom g = make_geom(l, b, kTokens, rows, scale_offset, span);
   const unsigned grid = (unsigned)(b.n * g.planes * g.chunks);
   if (max_grid > 0)
-    hipLaunchKernelGGL((fp8_save_linear<kLinearSaveBlock, kLinearSaveVecs, kScaleBf16, true, kTokens>),
-                       dim3(std::min((unsigned)max_grid, grid)), dim3(kLinearSaveBlock), 0, stream,
+    hipLaunchKernelGGL((fp8_save_linear<kSaveBlock, kSaveVecs, kScaleBf16, true, kTokens>),
+                       dim3(std::min((unsigned)max_grid, grid)), dim3(kSaveBlock), 0, stream,
                        (const uint16_t*)pool, g, rows, row_of, b);
   else
-    hipLaunchKernelGGL((fp8_save_linear<kLinearSaveBlock, kLinearSaveVecs, kScaleBf16, false, kTokens>), dim3(grid),
-                       dim3(kLinearSaveBlock), 0, stream, (const uint16_t*)pool, g, rows, row_of, b);
+    hipLaunchKernelGGL((fp8_save_linear<kSaveBlock, kSaveVecs, kScaleBf16, false, kTokens>), dim3(grid),
+                       dim3(kSaveBlock), 0, stream, (const uint16_t*)pool, g, rows, row_of, b);
   return hipGetLastError();
+}
+
+template <bool kScaleBf16, bool kTokens>
+static hipError_t launch_fp8_linear(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
+                                    int64_t scale_offset, int32_t max_grid, hipStream_t stream,
+                                    const TokenSpan* span) {
+  const int64_t row = l.head_dim / 8, plane = row * l.plane_rows;
+  if (!kTokens && max_grid <= 0 && row <= kLinearSmallBlock * kLinearSmallSaveVecs &&
+      (plane <= kLinearSmallPlane || plane * l.planes * b.n <= kLinearSmallTotal))
+    return launch_fp8_linear_as<kLinearSmallBlock, kLinearSmallSaveVecs, kLinearSmallBlock, kLinearSmallRestoreVecs,
+                                kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
+  return launch_fp8_linear_as<kLinearSaveBlock, kLinearSaveVecs, kLinearRestoreBlock, kLinearRestoreVecs, kScaleBf16,
+                              kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
 }
 
 template <bool kScaleBf16, bool kTokens>
@@ -1023,12 +1058,14 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
     return hipGetLastError();
   };
   // Rows of 64 fill half of a restore wave's code loads: only their striding
-  // kernels are used. The linear kernels restore 100 blocks of 64 x 1024 such
-  // rows in 210 us (245 here) and save them in 201 us (242).
-  const bool tuned = access == kVectorAccess && (l.head_dim != 64 || max_grid > 0);
+  // kernels and small saves are used. The linear kernels restore 100 blocks of
+  // 64 x 1024 such rows in 210 us (245 here) and save them in 201 us (242).
+  const int64_t rows = (int64_t)b.n * l.planes * l.plane_rows;
+  const bool tuned = access == kVectorAccess &&
+                     (l.head_dim != 64 || max_grid > 0 || (!kTokens && save && rows <= kTiledSave64Rows));
   switch (tuned ? l.head_dim : 0) {
     case 64:
-      return run(fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, true, kTokens>,
+      return run(fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, kTokens, kTokens>,
                  fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, true, kTokens>,
                  fp8_restore_kernel<64, 1, kRestoreStrideBlock, kScaleBf16, true, kTokens>,
                  fp8_restore_kernel<64, 1, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<64, 1>::kLanes);

@@ -24,6 +24,12 @@ def finite_pool(gpu, layers, blocks, bs, heads, hd, seed=0):
 WIDTHS = [(2, 63, 1, 96), (2, 64, 1, 96), (1, 65, 1, 96), (1, 256, 3, 96), (2, 73, 1, 80), (1, 49, 2, 112),
           (2, 33, 1, 192), (1, 300, 5, 8), (1, 97, 1, 16), (1, 77, 1, 40), (1, 3, 1, 6144), (1, 2, 1, 6152),
           (1, 5, 3, 100), (2, 49, 1, 128), (1, 17, 1, 256), (1, 200, 1, 64)]
+# The launches above are small ones, in one-wave workgroups of 128 pieces to save and 64 to restore (at most 196,608
+# pieces, here in 2 blocks). Larger: planes at and around whole tiles, of at most 192 pieces (one wave again) and just
+# above.
+WIDTHS += [(66, 64, 1, 96), (66, 65, 1, 96), (66, 800, 1, 8), (260, 24, 1, 64), (260, 25, 1, 64), (250, 16, 1, 96)]
+# Rows of 64 above the tiled kernel's 8,192 rows to save.
+WIDTHS += [(16, 130, 1, 64)]
 
 
 @pytest.mark.parametrize("shift", [0, 8])  # payloads 16-byte aligned, or only 8
