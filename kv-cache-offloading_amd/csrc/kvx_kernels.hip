@@ -569,15 +569,17 @@ __global__ __launch_bounds__(kBlock) void fp8_save_linear(const uint16_t* __rest
 }
 
 // Restore: needs no LDS, as each piece's scale is one (cached) load, and so no
-// whole rows per tile either: g.chunks tiles of kBlock * kVecs pieces cover a
+// whole rows per tile either: g.chunks tiles of tile_pieces pieces cover a
 // plane, wherever its rows begin (80 blocks of 64 x 2048 rows of 96: 505 us,
 // against 524 with whole rows per tile). Threads x pieces: 256 x 2 505,
 // 512 x 2 518, 128 x 4 543, 64 x 4 548, 256 x 3 586, 256 x 1 638.
 template <int kBlock, int kVecs, bool kScaleBf16, bool kTokens>
-__global__ __launch_bounds__(kBlock) void fp8_restore_linear(uint16_t* __restrict__ pool, PlaneGeom g, FastDiv row_of,
-                                                            BlockBatch b) {
-  const TileCoord tc = tile_coord<kTokens, kTokens ? kTokenRestoreOrder : kRestoreOrder>(g, kBlock * kVecs);  // row0 counts pieces here
-  const int pieces = (tc.entry == b.n - 1 ? g.last_rows : g.plane_rows) * (g.head_dim / 8);
+__global__ __launch_bounds__(kBlock) void fp8_restore_linear(uint16_t* __restrict__ pool, PlaneGeom g,
+                                                            int tile_pieces, FastDiv row_of, BlockBatch b) {
+  // row0 counts pieces here.
+  const TileCoord tc = tile_coord<kTokens, kTokens ? kTokenRestoreOrder : kRestoreOrder>(g, tile_pieces);
+  int pieces = (tc.entry == b.n - 1 ? g.last_rows : g.plane_rows) * (g.head_dim / 8);
+  pieces = min(pieces, tc.row0 + tile_pieces);
   uint16_t* dst = pool + (int64_t)b.ids[tc.entry] * g.block_stride + (int64_t)tc.plane * g.plane_stride;
   const uint8_t* payload =
       reinterpret_cast<const uint8_t*>(b.entries[tc.entry]) + (int64_t)tc.plane * g.payload_plane_stride;
@@ -982,6 +984,19 @@ constexpr int64_t kLinearSmallTotal = 192 << 10;
 // kernel, whose row maxima need no barrier: 2,048 rows 2.4 us (2.7 with the
 // linear one), 4,096 2.75 (2.9), 8,200 3.0 (3.0).
 constexpr int64_t kTiledSave64Rows = 8192;
+constexpr int kLinePieces = 16;  // 128 bytes of codes
+
+// Tiles of at most `most` items (a multiple of `step`) for a plane of `items`: of that size, unless the last one
+// would then be less than a quarter full, and of about equal size, in steps of `step`, if so. A nearly empty tile
+// costs almost a full one: 4,096 planes of 65 rows of 64 (520 pieces) restored in 15.5 us as 512 + 8, 12.1 us as
+// 272 + 248; 2,048 of 97 saved in 12.1 us as 96 + 1 rows, 9.5 as 50 + 47. Planes whose last tile is fuller gained
+// nothing (96 rows of 96 restored: 23.8 and 24.1).
+static int64_t spread(int64_t items, int64_t most, int64_t step) {
+  const int64_t last = items % most;
+  if (items <= most || last == 0 || last * 4 >= most) return most;
+  const int64_t tiles = items / most + 1, even = (items + tiles - 1) / tiles;
+  return (even + step - 1) / step * step;
+}
 
 template <int kSaveBlock, int kSaveVecs, int kRestoreBlock, int kRestoreVecs, bool kScaleBf16, bool kTokens>
 static hipError_t launch_fp8_linear_as(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
@@ -992,16 +1007,17 @@ static hipError_t launch_fp8_linear_as(bool save, void* pool, const kvx_block_la
   if (!save) {
     constexpr int kPieces = kRestoreBlock * kRestoreVecs;
     PlaneGeom g = make_geom(l, b, kTokens, 0, scale_offset, span);
-    set_chunks(g, ((int64_t)l.plane_rows * row_pieces + kPieces - 1) / kPieces);
+    const int64_t pieces = (int64_t)l.plane_rows * row_pieces, tile = spread(pieces, kPieces, kLinePieces);
+    set_chunks(g, (pieces + tile - 1) / tile);
     hipLaunchKernelGGL((fp8_restore_linear<kRestoreBlock, kRestoreVecs, kScaleBf16, kTokens>),
                        dim3((unsigned)(b.n * g.planes * g.chunks)), dim3(kRestoreBlock), 0, stream,
-                       (uint16_t*)pool, g, row_of, b);
+                       (uint16_t*)pool, g, (int)tile, row_of, b);
     return hipGetLastError();
   }
   // As many rows as fit, in whole 128-byte lines of codes (and of bf16) if any such number fits.
   const int32_t most = kSaveBlock * kSaveVecs / row_pieces;
   const int32_t lines = 128 / std::min(128, l.head_dim & -l.head_dim);
-  const int32_t rows = most >= lines ? most / lines * lines : most;
+  const int32_t rows = most >= lines ? (int32_t)spread(l.plane_rows, most / lines * lines, lines) : most;
   const PlaneGeom g = make_geom(l, b, kTokens, rows, scale_offset, span);
   const unsigned grid = (unsigned)(b.n * g.planes * g.chunks);
   if (max_grid > 0)

@@ -25,9 +25,10 @@ WIDTHS = [(2, 63, 1, 96), (2, 64, 1, 96), (1, 65, 1, 96), (1, 256, 3, 96), (2, 7
           (2, 33, 1, 192), (1, 300, 5, 8), (1, 97, 1, 16), (1, 77, 1, 40), (1, 3, 1, 6144), (1, 2, 1, 6152),
           (1, 5, 3, 100), (2, 49, 1, 128), (1, 17, 1, 256), (1, 200, 1, 64)]
 # The launches above are small ones, in one-wave workgroups of 128 pieces to save and 64 to restore (at most 196,608
-# pieces, here in 2 blocks). Larger: planes at and around whole tiles, of at most 192 pieces (one wave again) and just
-# above.
-WIDTHS += [(66, 64, 1, 96), (66, 65, 1, 96), (66, 800, 1, 8), (260, 24, 1, 64), (260, 25, 1, 64), (250, 16, 1, 96)]
+# pieces, here in 2 blocks). Larger: planes at and around whole tiles, a last tile spread over the others (65 and 97
+# rows of 64, 65 of 96, 800 of 8) and not (81 of 96), planes of at most 192 pieces (one wave again) and just above.
+WIDTHS += [(66, 64, 1, 96), (66, 65, 1, 96), (60, 81, 1, 96), (100, 65, 1, 64), (66, 97, 1, 64), (66, 800, 1, 8),
+           (260, 24, 1, 64), (260, 25, 1, 64), (250, 16, 1, 96)]
 # Rows of 64 above the tiled kernel's 8,192 rows to save.
 WIDTHS += [(16, 130, 1, 64)]
 
