@@ -607,7 +607,8 @@ __global__ __launch_bounds__(kBlock) void fp8_restore_linear(uint16_t* __restric
 // ---------------------------------------------------------------------------
 // FP8 save / restore, generic path (any head_dim and alignment): one thread per
 // row. Left for rows that 8-element pieces cannot cover (the reference tests'
-// head_dim 4) or address (pools that are not 16-byte aligned).
+// head_dim 4) or address (pools that are not 16-byte aligned), and for many
+// planes of a few narrow rows (narrow_planes).
 
 __device__ __forceinline__ bool generic_row(const PlaneGeom& g, int n, int64_t& entry, int64_t& plane,
                                             int64_t& row) {
@@ -998,6 +999,17 @@ static int64_t spread(int64_t items, int64_t most, int64_t step) {
   return (even + step - 1) / step * step;
 }
 
+// Many planes of a few narrow rows are left to the generic kernels: there the linear ones are bound by one
+// workgroup per plane, while a row of up to 24 elements is little work for one thread. Times in us, linear (one
+// wave) / generic: 65,536 planes of 8 rows of 8 saved 18.9 / 11.6 and restored 16.1 / 9.2, 262,144 of one row of 24
+// 64.6 / 34.2 and 57.8 / 42.0; at the lines 8,200 planes of 8 rows of 8 4.2 / 4.3 and 3.5 / 3.4, 16,384 of 2 rows of
+// 16 6.2 / 7.5 and 5.2 / 5.05, 262,144 of 4 rows of 16 67.6 / 72.0 and 57.7 / 50.7, of 2 of 24 66.9 / 69.5 and
+// 57.9 / 77.0.
+static bool narrow_planes(const kvx_block_layout& l, int32_t n) {
+  const int64_t row = l.head_dim / 8;
+  return l.head_dim % 8 == 0 && row * row * l.plane_rows <= 9 && (int64_t)l.planes * n > 8192 * row;
+}
+
 template <int kSaveBlock, int kSaveVecs, int kRestoreBlock, int kRestoreVecs, bool kScaleBf16, bool kTokens>
 static hipError_t launch_fp8_linear_as(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
                                        int64_t scale_offset, int32_t max_grid, hipStream_t stream,
@@ -1100,7 +1112,8 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
       // take rows of 128 and 256 too, but save 128 Qwen3-8B blocks in 1,131 us
       // against fp8_save_kernel's 1,085 and restore them in 1,158 against
       // fp8_restore_kernel's 1,143.
-      if (access != kAnyAccess && l.head_dim % 8 == 0 && l.head_dim / 8 <= kLinearMaxPieces)
+      if (access != kAnyAccess && l.head_dim % 8 == 0 && l.head_dim / 8 <= kLinearMaxPieces &&
+          (max_grid > 0 || !narrow_planes(l, b.n)))
         return launch_fp8_linear<kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
       PlaneGeom g = make_geom(l, b, kTokens, 0, scale_offset, span);
       const unsigned grid = generic_grid((int64_t)b.n * l.planes * l.plane_rows);

@@ -29,8 +29,9 @@ WIDTHS = [(2, 63, 1, 96), (2, 64, 1, 96), (1, 65, 1, 96), (1, 256, 3, 96), (2, 7
 # rows of 64, 65 of 96, 800 of 8) and not (81 of 96), planes of at most 192 pieces (one wave again) and just above.
 WIDTHS += [(66, 64, 1, 96), (66, 65, 1, 96), (60, 81, 1, 96), (100, 65, 1, 64), (66, 97, 1, 64), (66, 800, 1, 8),
            (260, 24, 1, 64), (260, 25, 1, 64), (250, 16, 1, 96)]
-# Rows of 64 above the tiled kernel's 8,192 rows to save.
-WIDTHS += [(16, 130, 1, 64)]
+# Rows of 64 above the tiled kernel's 8,192 rows to save. Many planes of a few narrow rows (above 8,192 per 8 elements
+# of the row), which one thread per row handles, and the same with a row more.
+WIDTHS += [(16, 130, 1, 64), (2060, 8, 1, 8), (2060, 9, 1, 8), (2060, 10, 1, 8), (4110, 2, 1, 16), (4110, 3, 1, 16)]
 
 
 @pytest.mark.parametrize("shift", [0, 8])  # payloads 16-byte aligned, or only 8
