@@ -61,10 +61,10 @@ struct PlaneGeom {
   int32_t last_rows;
   int32_t head_dim;
   int32_t scales16;      // every plane's scales start on 16 bytes (given 16-byte entries)
-  int32_t chunks;        // tiles per plane
-  FastDiv plane_of;      // tile -> plane of the batch (/ chunks)
-  int32_t inner;         // planes, or for token entries the entries of the batch
-  FastDiv outer_of;      // plane of the batch -> entry, or for token entries its plane (/ inner)
+  int32_t chunks;        // tiles per plane of an entry (fewer in the last of a batch of token entries)
+  int32_t outer_tiles;   // tiles per entry, or for token entries per plane over the entries of the batch
+  FastDiv outer_of;      // tile -> entry, or for token entries plane (/ outer_tiles)
+  FastDiv inner_of;      // tile of that -> plane, or for token entries entry (/ chunks)
 };
 
 // FP8 token entries of one launch (see PlaneGeom).

@@ -61,7 +61,9 @@ def test_fp8_blocks_of_any_row_width(gpu, layers, bs, heads, hd, scale_dtype, sh
 # Token counts whose planes of scales (and, with 3 heads of 40, of codes) are not multiples of 16 bytes.
 @pytest.mark.parametrize("scale_dtype", SCALES)
 @pytest.mark.parametrize("heads,hd,tokens", [(1, 128, 1), (1, 128, 257), (2, 128, 511), (1, 64, 513), (3, 40, 301),
-                                             (1, 256, 255), (3, 96, 512), (1, 112, 299)])
+                                             (1, 256, 255), (3, 96, 512), (1, 112, 299),
+                                             # the last block at, above and below whole tiles
+                                             (1, 128, 16), (1, 128, 273), (1, 256, 264), (1, 64, 352), (1, 96, 64)])
 def test_fp8_tokens_of_any_count_and_width(gpu, heads, hd, tokens, scale_dtype):
     pool = finite_pool(gpu, 2, 6, 256, heads, hd, seed=tokens)
     before = bf16_bits(pool)
@@ -76,6 +78,22 @@ def test_fp8_tokens_of_any_count_and_width(gpu, heads, hd, tokens, scale_dtype):
     assert np.array_equal(u8(scale).ravel(), scales.view(np.uint8).ravel())
     ops.scatter_tokens_fp8(pool, dest, tokens, payload, scale)
     oracle.scatter_tokens(before, dest, oracle.dequantize(codes, scales, fp32))
+    assert np.array_equal(bf16_bits(pool), before)
+
+
+# A tile is 1 KiB of a plane: the last block's share a fraction of one, whole ones, and one row more or less.
+@pytest.mark.parametrize("heads,hd,tokens", [(1, 128, 1), (1, 128, 4), (1, 128, 259), (1, 128, 260), (1, 128, 261),
+                                             (3, 40, 301), (2, 256, 512), (1, 8, 320)])
+def test_raw_tokens_of_any_count_and_width(gpu, heads, hd, tokens):
+    pool = finite_pool(gpu, 2, 6, 256, heads, hd, seed=tokens)
+    before = bf16_bits(pool)
+    table, dest = [4, 1, 2][:-(-tokens // 256)], [0, 5, 3][:-(-tokens // 256)]
+    dense = torch.empty((2, 2, tokens, heads, hd), dtype=torch.bfloat16, device=gpu)
+    ops.gather_tokens(pool, table, tokens, dense)
+    values = oracle.gather_tokens(before, table, tokens)
+    assert np.array_equal(bf16_bits(dense), values)
+    ops.scatter_tokens(pool, dest, tokens, dense)
+    oracle.scatter_tokens(before, dest, values)
     assert np.array_equal(bf16_bits(pool), before)
 
 
