@@ -147,6 +147,16 @@ __device__ __forceinline__ int xcd_tile(int bid, int grid) {
 constexpr int kSaveOrder = 8, kTokenSaveOrder = 6;
 constexpr int kRestoreOrder = kOrderEighths, kTokenRestoreOrder = kOrderDispatch;
 constexpr int kCopyOrder = 9, kTokenCopyOrder = kOrderDispatch;
+// Scatters of large planes in runs of 2^8 tiles. In the dispatcher's order all
+// XCDs write within a few KiB of the pool at a time, which is the fastest for
+// small planes and loses on large ones. Scattered with rows of 128 or 256, in us,
+// dispatcher's order / runs / one contiguous eighth per XCD (the order of the
+// entry-major copies before): 32 heads of 128, 256 tokens 43.6 / 37.4 / 39.7,
+// 20,000 tokens 3305 / 2811 / 2749; 8 heads of 256, 20,000 tokens 1537 / 1398 /
+// 1399; 8 of 128 721 / 700 / 716 and, 2,064 tokens, 72.4 / 72.5 / 77.2; 2 of 128,
+// 20,000 tokens, 172 / 175 / 184.
+constexpr int kTokenRestoreRuns = 8;
+constexpr int64_t kTokenRunPlane = 256 << 10;  // elements of a block's plane
 // Smaller copies leave no whole number of run rounds and keep the dispatcher's
 // order: 147,456 tiles (4 Qwen3-8B blocks each way) 98.4 us, 99.2 in runs of
 // 512; 294,912 tiles 184.0 and 181.9; 64 blocks of 72 x 1024 rows of 128
@@ -449,7 +459,8 @@ __global__ __launch_bounds__(kBlock) void fp8_save_kernel(const uint16_t* __rest
 // (one-wave workgroups; 128 and 256 threads gave ~6.48 and ~6.43).
 // kStride: restores read straight from host slots, by a capped grid whose
 // workgroups stride over the tiles (as the striding save instance).
-template <int kHd, int kVec, int kBlock, bool kScaleBf16, bool kStride, bool kTokens>
+template <int kHd, int kVec, int kBlock, bool kScaleBf16, bool kStride, bool kTokens,
+          int kOrder = kTokens ? kTokenRestoreOrder : kRestoreOrder>
 __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restrict__ pool, PlaneGeom g,
                                                             BlockBatch b) {
   using M = RowMap<kHd, kVec>;
@@ -459,7 +470,7 @@ __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restric
   const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
   for (int tile = kStride ? (int)blockIdx.x : 0; tile < tiles; tile += kStride ? (int)gridDim.x : 1) {
   if (kStride) __syncthreads();  // the previous tile's codes have been read back
-  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, kRows, tile) : tile_coord<kTokens, kTokens ? kTokenRestoreOrder : kRestoreOrder>(g, kRows);
+  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, kRows, tile) : tile_coord<kTokens, kOrder>(g, kRows);
   const int lane = threadIdx.x % M::kLanes;
   const int rsub = threadIdx.x / M::kLanes;
   const int row = tc.row0 + rsub;
@@ -1094,6 +1105,8 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
   const int64_t rows = (int64_t)b.n * l.planes * l.plane_rows;
   const bool tuned = access == kVectorAccess &&
                      (l.head_dim != 64 || max_grid > 0 || (!kTokens && save && rows <= kTiledSave64Rows));
+  constexpr int kRuns = kTokens ? kTokenRestoreRuns : kRestoreOrder;
+  const bool runs = kTokens && (int64_t)l.plane_rows * l.head_dim >= kTokenRunPlane;
   switch (tuned ? l.head_dim : 0) {
     case 64:
       return run(fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, kTokens, kTokens>,
@@ -1103,12 +1116,14 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
     case 128:
       return run(fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, false, kTokens>,
                  fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, true, kTokens>,
-                 fp8_restore_kernel<128, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
+                 runs ? fp8_restore_kernel<128, 2, kRestoreBlock, kScaleBf16, false, kTokens, kRuns>
+                      : fp8_restore_kernel<128, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
                  fp8_restore_kernel<128, 2, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<128, 2>::kLanes);
     case 256:
       return run(fp8_save_kernel<256, 2, kSaveBlock, kScaleBf16, false, kTokens>,
                  fp8_save_kernel<256, 2, kSaveBlock, kScaleBf16, true, kTokens>,
-                 fp8_restore_kernel<256, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
+                 runs ? fp8_restore_kernel<256, 2, kRestoreBlock, kScaleBf16, false, kTokens, kRuns>
+                      : fp8_restore_kernel<256, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
                  fp8_restore_kernel<256, 2, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<256, 2>::kLanes);
     default: {
       // Other widths, and payloads on 8 bytes only: the linear kernels. They

@@ -63,7 +63,9 @@ def test_fp8_blocks_of_any_row_width(gpu, layers, bs, heads, hd, scale_dtype, sh
 @pytest.mark.parametrize("heads,hd,tokens", [(1, 128, 1), (1, 128, 257), (2, 128, 511), (1, 64, 513), (3, 40, 301),
                                              (1, 256, 255), (3, 96, 512), (1, 112, 299),
                                              # the last block at, above and below whole tiles
-                                             (1, 128, 16), (1, 128, 273), (1, 256, 264), (1, 64, 352), (1, 96, 64)])
+                                             (1, 128, 16), (1, 128, 273), (1, 256, 264), (1, 64, 352), (1, 96, 64),
+                                             # planes scattered in runs of tiles per XCD
+                                             (8, 128, 700), (4, 256, 300)])
 def test_fp8_tokens_of_any_count_and_width(gpu, heads, hd, tokens, scale_dtype):
     pool = finite_pool(gpu, 2, 6, 256, heads, hd, seed=tokens)
     before = bf16_bits(pool)
