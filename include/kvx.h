@@ -47,7 +47,7 @@ extern "C" {
 #define KVX_OK 0
 #define KVX_E_INVALID (-1)  /* malformed argument (null pointer, bad size, bad layout) */
 #define KVX_E_RANGE (-2)    /* block id / slot / size outside its valid range */
-#define KVX_E_STATE (-3)    /* object in the wrong state (e.g. no staging attached) */
+#define KVX_E_STATE (-3)    /* object in the wrong state (e.g. no staging attached), or out of host memory */
 #define KVX_E_UNSUPPORTED (-4) /* valid request this build does not implement */
 
 /* Scale element types of an FP8 entry. */

@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <exception>
 #include <initializer_list>
 #include <mutex>
 #include <new>
@@ -28,6 +29,19 @@ int set_error(int code, const char* fmt, ...) {
 int hip_status(hipError_t err, const char* what) {
   if (err == hipSuccess) return KVX_OK;
   return set_error((int)err, "%s: %s (hipError_t %d)", what, hipGetErrorString(err), (int)err);
+}
+
+// Runs the part of a call that allocates host memory: no C++ exception may
+// leave a C function, whose callers (ctypes, C) cannot unwind one.
+template <typename F>
+static int no_throw(F body) {
+  try {
+    return body();
+  } catch (const std::bad_alloc&) {
+    return set_error(KVX_E_STATE, "out of host memory");
+  } catch (const std::exception& e) {
+    return set_error(KVX_E_STATE, "%s", e.what());
+  }
 }
 
 // No layout, tensor, entry run or slab this library addresses may span more
@@ -437,10 +451,18 @@ struct kvx_cache {
         delete e;
         return hip_status(err, "hipEventCreateWithFlags");
       }
-      all_events.push_back(e);
       // unref() returns events with push_back: with this capacity it never
       // reallocates, so calls that create no event allocate nothing.
-      free_events.reserve(all_events.size());
+      const int rc = no_throw([&] {
+        free_events.reserve(all_events.size() + 1);
+        all_events.push_back(e);
+        return KVX_OK;
+      });
+      if (rc) {
+        (void)hipEventDestroy(e->ev);
+        delete e;
+        return rc;
+      }
     }
     e->refs = 0;
     *out = e;
@@ -461,6 +483,14 @@ struct kvx_cache {
 
   void release_if_unused(Event* e) {
     if (e->refs == 0) free_events.push_back(e);
+  }
+
+  // Room for one more entry of caller_reads, so that track_caller_read cannot fail.
+  int reserve_caller_read() {
+    return no_throw([&] {
+      caller_reads.reserve(caller_reads.size() + 1);
+      return KVX_OK;
+    });
   }
 
   // Tracks `e`, just recorded on caller stream `s`, in place of the stream's
@@ -558,7 +588,13 @@ struct kvx_cache {
       if (slots[i] < 0 || slots[i] >= num_slots)
         return set_error(KVX_E_RANGE, "host slot %d outside [0, %d)", slots[i], num_slots);
     }
-    if (any_repeat(save ? slots : ids, n))
+    bool repeat = false;
+    const int rc = no_throw([&] {
+      repeat = any_repeat(save ? slots : ids, n);
+      return KVX_OK;
+    });
+    if (rc) return rc;
+    if (repeat)
       return set_error(KVX_E_INVALID, save ? "a slot appears twice in one save" : "a block appears twice in one restore");
     if (n > 0 && staged && !save_staging) return set_error(KVX_E_STATE, "no staging attached");
     return KVX_OK;
@@ -797,39 +833,51 @@ int kvx_store_kvcache(const void* key, int64_t key_stride, const void* value, in
 
 int kvx_save_blocks(const void* pool, const kvx_block_layout* layout, int32_t format, const int32_t* block_ids_host,
                     const uint64_t* entries_host, int32_t n, int64_t scale_offset, void* stream) {
-  return run_batches(true, const_cast<void*>(pool), layout, format, block_ids_host, entries_host, n, scale_offset,
-                     (hipStream_t)stream);
+  return no_throw([&] {
+    return run_batches(true, const_cast<void*>(pool), layout, format, block_ids_host, entries_host, n, scale_offset,
+                       (hipStream_t)stream);
+  });
 }
 
 int kvx_restore_blocks(void* pool, const kvx_block_layout* layout, int32_t format, const int32_t* block_ids_host,
                        const uint64_t* entries_host, int32_t n, int64_t scale_offset, void* stream) {
-  return run_batches(false, pool, layout, format, block_ids_host, entries_host, n, scale_offset,
-                     (hipStream_t)stream);
+  return no_throw([&] {
+    return run_batches(false, pool, layout, format, block_ids_host, entries_host, n, scale_offset,
+                       (hipStream_t)stream);
+  });
 }
 
 int kvx_gather_tokens(const void* pool, const kvx_block_layout* layout, const int32_t* block_table_host,
                       int32_t table_len, int64_t num_rows, void* dst, void* stream) {
-  return token_copy(true, const_cast<void*>(pool), layout, block_table_host, table_len, num_rows, dst,
-                    (hipStream_t)stream);
+  return no_throw([&] {
+    return token_copy(true, const_cast<void*>(pool), layout, block_table_host, table_len, num_rows, dst,
+                      (hipStream_t)stream);
+  });
 }
 
 int kvx_scatter_tokens(void* pool, const kvx_block_layout* layout, const int32_t* block_table_host,
                        int32_t table_len, int64_t num_rows, const void* src, void* stream) {
-  return token_copy(false, pool, layout, block_table_host, table_len, num_rows, const_cast<void*>(src),
-                    (hipStream_t)stream);
+  return no_throw([&] {
+    return token_copy(false, pool, layout, block_table_host, table_len, num_rows, const_cast<void*>(src),
+                      (hipStream_t)stream);
+  });
 }
 
 int kvx_gather_tokens_fp8(const void* pool, const kvx_block_layout* layout, const int32_t* block_table_host,
                           int32_t table_len, int64_t num_rows, void* payload, void* scales, void* stream) {
-  return token_fp8(true, const_cast<void*>(pool), layout, block_table_host, table_len, num_rows, payload, scales,
-                   (hipStream_t)stream);
+  return no_throw([&] {
+    return token_fp8(true, const_cast<void*>(pool), layout, block_table_host, table_len, num_rows, payload, scales,
+                     (hipStream_t)stream);
+  });
 }
 
 int kvx_scatter_tokens_fp8(void* pool, const kvx_block_layout* layout, const int32_t* block_table_host,
                            int32_t table_len, int64_t num_rows, const void* payload, const void* scales,
                            void* stream) {
-  return token_fp8(false, pool, layout, block_table_host, table_len, num_rows, const_cast<void*>(payload),
-                   const_cast<void*>(scales), (hipStream_t)stream);
+  return no_throw([&] {
+    return token_fp8(false, pool, layout, block_table_host, table_len, num_rows, const_cast<void*>(payload),
+                     const_cast<void*>(scales), (hipStream_t)stream);
+  });
 }
 
 int kvx_upload(void* dst, const void* src_pinned, int64_t nbytes, void* stream) {
@@ -898,8 +946,15 @@ int kvx_cache_create(void* pool, const kvx_block_layout* layout, int32_t format,
   // Host slots are 256-byte aligned and entry_stride apart (a multiple of 256),
   // so the pool alone decides whether the vector kernels can address them.
   c->host_reads_ok = striding_restore_supported(*layout, format, access_of(pool, *layout, nullptr, 0));
-  c->pending_save.assign(layout->num_blocks, nullptr);
-  c->pending_restore.assign(layout->num_blocks, nullptr);
+  rc = no_throw([&] {
+    c->pending_save.assign(layout->num_blocks, nullptr);
+    c->pending_restore.assign(layout->num_blocks, nullptr);
+    return KVX_OK;
+  });
+  if (rc) {
+    delete c;  // nothing is queued on the caller's streams yet
+    return rc;
+  }
   DeviceScope scope;
   rc = scope.enter(device);
   // The marker only orders device work behind device work: saves behind the
@@ -986,11 +1041,15 @@ int kvx_cache_add_slab(kvx_cache* c, void* host_base, int32_t count) {
   int64_t slab_bytes;
   if (!span_product({count, c->entry_stride}, &slab_bytes))
     return set_error(KVX_E_UNSUPPORTED, "a slab of %d entries spans more than 2^40 bytes", count);
-  c->slabs.push_back(Slab{(uint8_t*)host_base, c->num_slots, count});
-  c->num_slots += count;
-  c->slot_read.resize(c->num_slots, nullptr);
-  c->slot_saved.resize(c->num_slots, nullptr);
-  return KVX_OK;
+  return no_throw([&] {
+    const int32_t slots = c->num_slots + count;
+    // The slots exist once num_slots counts them, after the last allocation.
+    c->slot_read.resize(slots, nullptr);
+    c->slot_saved.resize(slots, nullptr);
+    c->slabs.push_back(Slab{(uint8_t*)host_base, c->num_slots, count});
+    c->num_slots = slots;
+    return KVX_OK;
+  });
 }
 
 int kvx_cache_reset_slabs(kvx_cache* c) {
@@ -1071,6 +1130,7 @@ int kvx_cache_restore(kvx_cache* c, const int32_t* slots, const int32_t* ids, in
   // per call on MI355X, against ~5 us for the launch.
   const bool direct = c->direct_restore(n, wait != 0);
   hipStream_t s = direct ? compute : c->restore_stream;
+  if (s == compute && (rc = c->reserve_caller_read())) return rc;
   // What the work of blocks [base, base + cnt) waits for on `s`. With the
   // restore on the save stream (one copy stream), stream order covers saves.
   const bool order_saves = c->split || s != c->save_stream;
