@@ -46,13 +46,24 @@ int scale_code(at::ScalarType t) {
   return t == at::kBFloat16 ? KVX_SCALE_BF16 : t == at::kFloat ? KVX_SCALE_FP32 : -1;
 }
 
+// Lets other Python threads run for the scope's lifetime, also if it is left by an exception.
+class WithoutGil {
+ public:
+  WithoutGil() : state_(PyEval_SaveThread()) {}
+  ~WithoutGil() { PyEval_RestoreThread(state_); }
+
+ private:
+  PyThreadState* state_;
+};
+
 // Runs `call` (a libkvx status) without the GIL: a launch may block on a full queue.
 template <typename F>
 PyObject* status(F call) {
   int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = call();
-  Py_END_ALLOW_THREADS;
+  {
+    WithoutGil released;
+    rc = call();
+  }
   return PyLong_FromLong(rc);
 }
 
