@@ -37,41 +37,43 @@ def hipcc() -> str:
 
 
 def build(arch: str = "gfx950", verbose: bool = False) -> Path:
-    cmd = [hipcc(), f"--offload-arch={arch}", *FLAGS, f"-I{ROOT / 'include'}", f"-I{HERE / 'csrc'}",
-           *map(str, SOURCES), "-o", str(OUTPUT) + ".tmp"]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    _run(cmd, OUTPUT, verbose)
-    build_bind(verbose)
+    """Compiles both, then puts both in place: a failed step leaves the pair that was there."""
+    _run([hipcc(), f"--offload-arch={arch}", *FLAGS, f"-I{ROOT / 'include'}", f"-I{HERE / 'csrc'}",
+          *map(str, SOURCES), "-o", _tmp(OUTPUT)], verbose)
+    _run(_bind_command(), verbose)
+    for output in (OUTPUT, BIND_OUTPUT):
+        os.replace(_tmp(output), output)
     return OUTPUT
 
 
-def build_bind(verbose: bool = False) -> Path:
+def _bind_command() -> list[str]:
     """kvx/_bind.so: host code only, against the installed torch's headers; it calls libkvx by address."""
     import sysconfig
 
     import torch
 
     torch_dir = Path(torch.__file__).parent
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
-           "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{ROOT / 'include'}",
-           f"-isystem{torch_dir / 'include'}", "-isystem/opt/rocm/include",
-           f"-I{sysconfig.get_paths()['include']}", str(BIND_SOURCE), "-o", str(BIND_OUTPUT) + ".tmp",
-           f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+            "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DKVX_TORCH_VERSION="{torch.__version__}"', f"-I{ROOT / 'include'}",
+            f"-isystem{torch_dir / 'include'}", "-isystem/opt/rocm/include",
+            f"-I{sysconfig.get_paths()['include']}", str(BIND_SOURCE), "-o", _tmp(BIND_OUTPUT),
+            f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
+def _tmp(output: Path) -> str:
+    return str(output) + ".tmp"
+
+
+def _run(cmd: list[str], verbose: bool):
     if verbose:
         print(" ".join(cmd), flush=True)
-    _run(cmd, BIND_OUTPUT, verbose)
-    return BIND_OUTPUT
-
-
-def _run(cmd: list[str], output: Path, verbose: bool):
     result = subprocess.run(cmd, capture_output=True, text=True, env=dict(os.environ))
     if result.returncode != 0:
         sys.stderr.write(result.stdout + result.stderr)
         raise RuntimeError(f"{cmd[0]} failed with exit code {result.returncode}")
     if verbose and result.stderr.strip():
         sys.stderr.write(result.stderr)
-    os.replace(str(output) + ".tmp", output)
 
 
 def main():
