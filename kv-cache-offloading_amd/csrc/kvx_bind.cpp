@@ -230,4 +230,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_bind", nullptr, -1, methods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__bind() { return PyModule_Create(&module); }
+// ABI_VERSION: of the kvx.h it was compiled against; TORCH_VERSION: the torch whose tensors it reads.
+PyMODINIT_FUNC PyInit__bind() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && (PyModule_AddIntConstant(m, "ABI_VERSION", KVX_ABI_VERSION) ||
+            PyModule_AddStringConstant(m, "TORCH_VERSION", KVX_TORCH_VERSION))) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -4,14 +4,17 @@ torch is imported first on purpose: libkvx links the HIP runtime by its
 SONAME (libamdhip64.so.7), so loading it after torch binds it to the runtime
 torch already loaded and streams/pointers from torch are valid in libkvx.
 There is no fallback: if the library is missing or fails to load, every
-entry point raises.
+entry point raises. Only the native binding of the operators' common calls is
+optional: without it they call the same library from here.
 """
 
 import ctypes
+import importlib
 import threading
+import warnings
 from pathlib import Path
 
-import torch  # noqa: F401  (must precede the dlopen below)
+import torch  # must precede the dlopen below
 
 LIB_PATH = Path(__file__).resolve().with_name("libkvx.so")
 ABI_VERSION = 2
@@ -124,21 +127,43 @@ def lib() -> ctypes.CDLL:
 _bind = None
 
 
-def bind():
-    """The native operator binding (kvx/_bind.so, csrc/kvx_bind.cpp), calling the loaded libkvx. Raises if not built.
+def load_bind():
+    """The native operator binding (kvx/_bind.so, csrc/kvx_bind.cpp), calling the loaded libkvx.
 
-    Each of its functions returns libkvx's status, or None for a call it does not take."""
+    Each of its functions returns libkvx's status, or None for a call it does not take. Raises ImportError if it is
+    not built, or was built for another torch, and RuntimeError if it was built for another libkvx."""
+    handle = lib()
+    module = importlib.import_module("kvx._bind")
+    if module.ABI_VERSION != ABI_VERSION:
+        raise RuntimeError(f"kvx._bind was built for libkvx ABI {module.ABI_VERSION}, not {ABI_VERSION}: "
+                           "rebuild it with python kv-cache-offloading_amd/build.py")
+    if module.TORCH_VERSION != torch.__version__:
+        raise ImportError(f"kvx._bind was built for torch {module.TORCH_VERSION}, not {torch.__version__}")
+    module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
+        handle.kvx_store_kvcache, handle.kvx_save_blocks, handle.kvx_restore_blocks, handle.kvx_entry_layout)))
+    return module
+
+
+class _NoBind:
+    """Takes no call, so that every operator makes its checks and calls libkvx through ctypes."""
+
+    @staticmethod
+    def store(*args):
+        return None
+
+    codec = blocks = store
+
+
+def bind():
+    """load_bind's module, kept; without one for this torch, with one warning, a stand-in that takes no call."""
     global _bind
     if _bind is None:
-        handle = lib()
         try:
-            from kvx import _bind as module
+            _bind = load_bind()
         except ImportError as e:
-            raise RuntimeError(f"kvx._bind is not built for this torch ({e}): run "
-                               "python kv-cache-offloading_amd/build.py") from e
-        module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
-            handle.kvx_store_kvcache, handle.kvx_save_blocks, handle.kvx_restore_blocks, handle.kvx_entry_layout)))
-        _bind = module
+            warnings.warn(f"operators call libkvx through ctypes, which takes about 4 us more a call ({e}): run "
+                          "python kv-cache-offloading_amd/build.py", RuntimeWarning, stacklevel=3)
+            _bind = _NoBind
     return _bind
 
 

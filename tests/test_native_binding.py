@@ -1,11 +1,45 @@
-"""Building the library and its native operator binding, without a device."""
+"""Loading and building the native operator binding, without a device."""
 
 import importlib.util
+import sys
 from types import SimpleNamespace
 
 import pytest
+import torch
 
 from conftest import ROOT
+from kvx import _lib
+
+
+def bind_with(monkeypatch, module):
+    """_lib.bind() where importing kvx._bind gives `module` (None: not built)."""
+    monkeypatch.setitem(sys.modules, "kvx._bind", module)
+    monkeypatch.setattr(_lib, "_bind", None)
+    return _lib.bind()
+
+
+def test_the_built_binding_matches_the_library_and_this_torch():
+    module = _lib.load_bind()
+    assert (module.ABI_VERSION, module.TORCH_VERSION) == (_lib.ABI_VERSION, torch.__version__)
+
+
+def test_operators_run_through_ctypes_without_a_binding(monkeypatch):
+    with pytest.warns(RuntimeWarning, match="ctypes"):
+        binding = bind_with(monkeypatch, None)
+    assert binding.store() is None and binding.codec() is None and binding.blocks() is None
+    assert _lib.bind() is binding  # one warning only
+
+
+def test_a_binding_of_another_torch_is_not_used(monkeypatch):
+    other = SimpleNamespace(ABI_VERSION=_lib.ABI_VERSION, TORCH_VERSION="0.0")
+    with pytest.warns(RuntimeWarning, match="built for torch 0.0"):
+        assert bind_with(monkeypatch, other).store() is None
+
+
+def test_a_binding_of_another_libkvx_is_refused(monkeypatch):
+    other = SimpleNamespace(ABI_VERSION=_lib.ABI_VERSION - 1, TORCH_VERSION=torch.__version__)
+    with pytest.raises(RuntimeError, match="ABI"):
+        bind_with(monkeypatch, other)
 
 
 def test_a_failed_build_leaves_the_pair_that_was_there(monkeypatch, tmp_path):
