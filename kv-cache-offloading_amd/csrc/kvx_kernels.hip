@@ -146,7 +146,7 @@ __device__ __forceinline__ int xcd_tile(int bid, int grid) {
 
 constexpr int kSaveOrder = 8, kTokenSaveOrder = 6;
 constexpr int kRestoreOrder = kOrderEighths, kTokenRestoreOrder = kOrderDispatch;
-constexpr int kCopyOrder = 9, kTokenCopyOrder = kOrderDispatch;
+constexpr int kCopyOrder = 9;
 // Scatters of large planes in runs of 2^8 tiles. In the dispatcher's order all
 // XCDs write within a few KiB of the pool at a time, which is the fastest for
 // small planes and loses on large ones. Scattered with rows of 128 or 256, in us,
@@ -403,12 +403,13 @@ __global__ __launch_bounds__(kBlock) void fp8_save_kernel(const uint16_t* __rest
   constexpr int kRows = kBlock / M::kLanes;       // rows per tile
   constexpr int kScaleBytes = kScaleBf16 ? 2 : 4;
   static_assert((kRows * kHd) % 16 == 0 && (kRows * kScaleBytes) % 16 == 0, "tile must store in 16-byte units");
+  constexpr int kOrder = kTokens ? kTokenSaveOrder : kSaveOrder;
   __shared__ uint4 codes[kRows * kHd / 16];
   __shared__ uint4 scale_tile[kRows * kScaleBytes / 16];
-  const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
+  const int tiles = kStride ? b.n * g.outer_tiles : 1;
   for (int tile = kStride ? (int)blockIdx.x : 0; tile < tiles; tile += kStride ? (int)gridDim.x : 1) {
   if (kStride) __syncthreads();  // the previous tile's stores have read the LDS tile
-  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, kRows, tile) : tile_coord<kTokens, kTokens ? kTokenSaveOrder : kSaveOrder>(g, kRows);
+  const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, kRows, tile) : tile_coord<kTokens, kOrder>(g, kRows);
   const int lane = threadIdx.x % M::kLanes;
   const int rsub = threadIdx.x / M::kLanes;
   const int row = tc.row0 + rsub;
@@ -459,15 +460,14 @@ __global__ __launch_bounds__(kBlock) void fp8_save_kernel(const uint16_t* __rest
 // (one-wave workgroups; 128 and 256 threads gave ~6.48 and ~6.43).
 // kStride: restores read straight from host slots, by a capped grid whose
 // workgroups stride over the tiles (as the striding save instance).
-template <int kHd, int kVec, int kBlock, bool kScaleBf16, bool kStride, bool kTokens,
-          int kOrder = kTokens ? kTokenRestoreOrder : kRestoreOrder>
+template <int kHd, int kVec, int kBlock, bool kScaleBf16, bool kStride, bool kTokens, int kOrder>
 __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restrict__ pool, PlaneGeom g,
                                                             BlockBatch b) {
   using M = RowMap<kHd, kVec>;
   constexpr int kRows = kBlock / M::kLanes;  // rows per tile
   constexpr int kPieces = kRows * kHd / 16;  // 16-byte pieces of the tile's codes
   __shared__ uint4 codes[kPieces];
-  const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
+  const int tiles = kStride ? b.n * g.outer_tiles : 1;
   for (int tile = kStride ? (int)blockIdx.x : 0; tile < tiles; tile += kStride ? (int)gridDim.x : 1) {
   if (kStride) __syncthreads();  // the previous tile's codes have been read back
   const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, kRows, tile) : tile_coord<kTokens, kOrder>(g, kRows);
@@ -531,11 +531,13 @@ template <int kBlock, int kVecs, bool kScaleBf16, bool kStride, bool kTokens>
 __global__ __launch_bounds__(kBlock) void fp8_save_linear(const uint16_t* __restrict__ pool, PlaneGeom g,
                                                          int tile_rows, FastDiv row_of, BlockBatch b) {
   constexpr int kPieces = kBlock * kVecs;
+  constexpr int kOrder = kTokens ? kTokenSaveOrder : kSaveOrder;
   __shared__ uint32_t row_max[kPieces];  // a tile of the narrowest rows (one piece each) has kPieces of them
   __shared__ float2 row_params[kPieces];
-  const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
+  const int tiles = kStride ? b.n * g.outer_tiles : 1;
   for (int tile = kStride ? (int)blockIdx.x : 0; tile < tiles; tile += kStride ? (int)gridDim.x : 1) {
-    const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, tile_rows, tile) : tile_coord<kTokens, kTokens ? kTokenSaveOrder : kSaveOrder>(g, tile_rows);
+    const TileCoord tc =
+        kStride ? tile_coord_at<kTokens>(g, tile_rows, tile) : tile_coord<kTokens, kOrder>(g, tile_rows);
     const int left = (tc.entry == b.n - 1 ? g.last_rows : g.plane_rows) - tc.row0;
     const int rows = left < tile_rows ? left : tile_rows;  // at most 0 past the end of a partial entry
     const int pieces = rows * (g.head_dim / 8);
@@ -710,7 +712,7 @@ __global__ __launch_bounds__(kBlock) void raw_copy_kernel(uint8_t* __restrict__ 
                                                          int64_t last_bytes) {
   constexpr int kVecs = kStride ? kStrideCopyVecs : kCopyVecs;
   constexpr int kTileBytes = kBlock * kVecs * 16;
-  const int tiles = kStride ? b.n * g.planes * g.chunks : 1;
+  const int tiles = kStride ? b.n * g.outer_tiles : 1;
   for (int t = kStride ? (int)blockIdx.x : 0; t < tiles; t += kStride ? (int)gridDim.x : 1) {
   const TileCoord tc = kStride ? tile_coord_at<kTokens>(g, 1, t) : tile_coord<kTokens, kOrder>(g, 1);
   const int e = tc.entry, p = tc.plane;
@@ -1046,13 +1048,16 @@ static hipError_t launch_fp8_linear_as(bool save, void* pool, const kvx_block_la
   const int32_t rows = most >= lines ? (int32_t)spread(l.plane_rows, most / lines * lines, lines) : most;
   PlaneGeom g = make_geom(l, scale_offset, span);
   const unsigned grid = set_tiles(g, b.n, kTokens, g.plane_rows, g.last_rows, rows);
-  if (max_grid > 0)
-    hipLaunchKernelGGL((fp8_save_linear<kSaveBlock, kSaveVecs, kScaleBf16, true, kTokens>),
-                       dim3(std::min((unsigned)max_grid, grid)), dim3(kSaveBlock), 0, stream,
-                       (const uint16_t*)pool, g, rows, row_of, b);
-  else
-    hipLaunchKernelGGL((fp8_save_linear<kSaveBlock, kSaveVecs, kScaleBf16, false, kTokens>), dim3(grid),
-                       dim3(kSaveBlock), 0, stream, (const uint16_t*)pool, g, rows, row_of, b);
+  if constexpr (!kTokens) {
+    if (max_grid > 0) {
+      hipLaunchKernelGGL((fp8_save_linear<kSaveBlock, kSaveVecs, kScaleBf16, true, false>),
+                         dim3(std::min((unsigned)max_grid, grid)), dim3(kSaveBlock), 0, stream,
+                         (const uint16_t*)pool, g, rows, row_of, b);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((fp8_save_linear<kSaveBlock, kSaveVecs, kScaleBf16, false, kTokens>), dim3(grid),
+                     dim3(kSaveBlock), 0, stream, (const uint16_t*)pool, g, rows, row_of, b);
   return hipGetLastError();
 }
 
@@ -1069,81 +1074,90 @@ static hipError_t launch_fp8_linear(bool save, void* pool, const kvx_block_layou
                               kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
 }
 
+// The tiled kernels, for kHd-wide rows. Workgroup sizes chosen by sweeps on the
+// Qwen3-8B block workload: save 128 threads (16 rows for hd=128), restore 64
+// threads (8 rows). A capped (striding) restore reads host slots and needs more
+// bytes in flight per workgroup: 256 threads (32 rows). Only launches for block
+// entries are capped. Rows of 64 have no uncapped restore.
+template <int kHd, int kVec, bool kScaleBf16, bool kTokens>
+static hipError_t launch_fp8_tiled(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
+                                   int64_t scale_offset, int32_t max_grid, hipStream_t stream,
+                                   const TokenSpan* span) {
+  constexpr int kSaveBlock = 128;
+  constexpr int kRestoreBlock = 64;
+  constexpr int kRestoreStrideBlock = 256;
+  constexpr int kLanes = RowMap<kHd, kVec>::kLanes;
+  const uint16_t* src = (const uint16_t*)pool;
+  uint16_t* dst = (uint16_t*)pool;
+  PlaneGeom g = make_geom(l, scale_offset, span);
+  auto tiles_of = [&](int block) {
+    return set_tiles(g, b.n, kTokens, g.plane_rows, g.last_rows, block / kLanes);
+  };
+  if constexpr (!kTokens) {
+    const unsigned cap = (unsigned)std::max(max_grid, 0);
+    if (cap > 0 && !save) {
+      const unsigned grid = std::min(cap, tiles_of(kRestoreStrideBlock));
+      hipLaunchKernelGGL((fp8_restore_kernel<kHd, kVec, kRestoreStrideBlock, kScaleBf16, true, false, kRestoreOrder>),
+                         dim3(grid), dim3(kRestoreStrideBlock), 0, stream, dst, g, b);
+      return hipGetLastError();
+    }
+    if (cap > 0 && cap < tiles_of(kSaveBlock)) {
+      hipLaunchKernelGGL((fp8_save_kernel<kHd, kVec, kSaveBlock, kScaleBf16, true, false>), dim3(cap),
+                         dim3(kSaveBlock), 0, stream, src, g, b);
+      return hipGetLastError();
+    }
+  }
+  if (save) {
+    const unsigned grid = tiles_of(kSaveBlock);
+    hipLaunchKernelGGL((fp8_save_kernel<kHd, kVec, kSaveBlock, kScaleBf16, false, kTokens>), dim3(grid),
+                       dim3(kSaveBlock), 0, stream, src, g, b);
+    return hipGetLastError();
+  }
+  if constexpr (kHd == 64) {
+    return hipErrorInvalidValue;
+  } else {
+    constexpr int kOrder = kTokens ? kTokenRestoreOrder : kRestoreOrder;
+    constexpr int kRuns = kTokens ? kTokenRestoreRuns : kRestoreOrder;
+    auto kernel = kTokens && (int64_t)l.plane_rows * l.head_dim >= kTokenRunPlane
+                      ? fp8_restore_kernel<kHd, kVec, kRestoreBlock, kScaleBf16, false, kTokens, kRuns>
+                      : fp8_restore_kernel<kHd, kVec, kRestoreBlock, kScaleBf16, false, kTokens, kOrder>;
+    const unsigned grid = tiles_of(kRestoreBlock);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kRestoreBlock), 0, stream, dst, g, b);
+    return hipGetLastError();
+  }
+}
+
 template <bool kScaleBf16, bool kTokens>
 static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, const BlockBatch& b,
                              int64_t scale_offset, Access access, int32_t max_grid, hipStream_t stream,
                              const TokenSpan* span = nullptr) {
-  // Workgroup sizes chosen by sweeps on the Qwen3-8B block workload: save
-  // 128 threads (16 rows for hd=128), restore 64 threads (8 rows). A capped
-  // (striding) restore reads host slots and needs more bytes in flight per
-  // workgroup: 256 threads (32 rows).
-  constexpr int kSaveBlock = 128;
-  constexpr int kRestoreBlock = 64;
-  constexpr int kRestoreStrideBlock = 256;
-  auto run = [&](auto save_k, auto save_stride_k, auto restore_k, auto restore_stride_k, int lanes) -> hipError_t {
-    const int block = save ? kSaveBlock : kRestoreBlock;
-    PlaneGeom g = make_geom(l, scale_offset, span);
-    const unsigned grid = set_tiles(g, b.n, kTokens, g.plane_rows, g.last_rows, block / lanes);
-    if (save && max_grid > 0 && (unsigned)max_grid < grid) {
-      hipLaunchKernelGGL(save_stride_k, dim3((unsigned)max_grid), dim3(kSaveBlock), 0, stream, (const uint16_t*)pool,
-                         g, b);
-    } else if (save) {
-      hipLaunchKernelGGL(save_k, dim3(grid), dim3(kSaveBlock), 0, stream, (const uint16_t*)pool, g, b);
-    } else if (max_grid > 0) {
-      PlaneGeom gs = make_geom(l, scale_offset, span);
-      const unsigned tiles = set_tiles(gs, b.n, kTokens, gs.plane_rows, gs.last_rows, kRestoreStrideBlock / lanes);
-      hipLaunchKernelGGL(restore_stride_k, dim3((unsigned)max_grid < tiles ? (unsigned)max_grid : tiles), dim3(kRestoreStrideBlock), 0,
-                         stream, (uint16_t*)pool, gs, b);
-    } else {
-      hipLaunchKernelGGL(restore_k, dim3(grid), dim3(kRestoreBlock), 0, stream, (uint16_t*)pool, g, b);
-    }
-    return hipGetLastError();
-  };
+  if (access == kVectorAccess && l.head_dim == 128)
+    return launch_fp8_tiled<128, 2, kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
+  if (access == kVectorAccess && l.head_dim == 256)
+    return launch_fp8_tiled<256, 2, kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
   // Rows of 64 fill half of a restore wave's code loads: only their striding
   // kernels and small saves are used. The linear kernels restore 100 blocks of
-  // 64 x 1024 such rows in 210 us (245 here) and save them in 201 us (242).
-  const int64_t rows = (int64_t)b.n * l.planes * l.plane_rows;
-  const bool tuned = access == kVectorAccess &&
-                     (l.head_dim != 64 || max_grid > 0 || (!kTokens && save && rows <= kTiledSave64Rows));
-  constexpr int kRuns = kTokens ? kTokenRestoreRuns : kRestoreOrder;
-  const bool runs = kTokens && (int64_t)l.plane_rows * l.head_dim >= kTokenRunPlane;
-  switch (tuned ? l.head_dim : 0) {
-    case 64:
-      return run(fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, kTokens, kTokens>,
-                 fp8_save_kernel<64, 1, kSaveBlock, kScaleBf16, true, kTokens>,
-                 fp8_restore_kernel<64, 1, kRestoreStrideBlock, kScaleBf16, true, kTokens>,
-                 fp8_restore_kernel<64, 1, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<64, 1>::kLanes);
-    case 128:
-      return run(fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, false, kTokens>,
-                 fp8_save_kernel<128, 2, kSaveBlock, kScaleBf16, true, kTokens>,
-                 runs ? fp8_restore_kernel<128, 2, kRestoreBlock, kScaleBf16, false, kTokens, kRuns>
-                      : fp8_restore_kernel<128, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
-                 fp8_restore_kernel<128, 2, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<128, 2>::kLanes);
-    case 256:
-      return run(fp8_save_kernel<256, 2, kSaveBlock, kScaleBf16, false, kTokens>,
-                 fp8_save_kernel<256, 2, kSaveBlock, kScaleBf16, true, kTokens>,
-                 runs ? fp8_restore_kernel<256, 2, kRestoreBlock, kScaleBf16, false, kTokens, kRuns>
-                      : fp8_restore_kernel<256, 2, kRestoreBlock, kScaleBf16, false, kTokens>,
-                 fp8_restore_kernel<256, 2, kRestoreStrideBlock, kScaleBf16, true, kTokens>, RowMap<256, 2>::kLanes);
-    default: {
-      // Other widths, and payloads on 8 bytes only: the linear kernels. They
-      // take rows of 128 and 256 too, but save 128 Qwen3-8B blocks in 1,131 us
-      // against fp8_save_kernel's 1,085 and restore them in 1,158 against
-      // fp8_restore_kernel's 1,143.
-      if (access != kAnyAccess && l.head_dim % 8 == 0 && l.head_dim / 8 <= kLinearMaxPieces &&
-          (max_grid > 0 || !narrow_planes(l, b.n)))
-        return launch_fp8_linear<kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
-      const PlaneGeom g = make_geom(l, scale_offset, span);
-      const unsigned grid = generic_grid((int64_t)b.n * l.planes * l.plane_rows);
-      if (save)
-        hipLaunchKernelGGL(fp8_save_generic<kScaleBf16>, dim3(grid), dim3(kThreads), 0, stream,
-                           (const uint16_t*)pool, g, b);
-      else
-        hipLaunchKernelGGL(fp8_restore_generic<kScaleBf16>, dim3(grid), dim3(kThreads), 0, stream,
-                           (uint16_t*)pool, g, b);
-      return hipGetLastError();
-    }
+  // 64 x 1024 such rows in 210 us (245 in tiled ones) and save them in 201 us (242).
+  if constexpr (!kTokens) {
+    const bool small_save = save && (int64_t)b.n * l.planes * l.plane_rows <= kTiledSave64Rows;
+    if (access == kVectorAccess && l.head_dim == 64 && (max_grid > 0 || small_save))
+      return launch_fp8_tiled<64, 1, kScaleBf16, false>(save, pool, l, b, scale_offset, max_grid, stream, span);
   }
+  // Other widths, and payloads on 8 bytes only: the linear kernels. They
+  // take rows of 128 and 256 too, but save 128 Qwen3-8B blocks in 1,131 us
+  // against fp8_save_kernel's 1,085 and restore them in 1,158 against
+  // fp8_restore_kernel's 1,143.
+  if (access != kAnyAccess && l.head_dim % 8 == 0 && l.head_dim / 8 <= kLinearMaxPieces &&
+      (max_grid > 0 || !narrow_planes(l, b.n)))
+    return launch_fp8_linear<kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
+  const PlaneGeom g = make_geom(l, scale_offset, span);
+  const unsigned grid = generic_grid((int64_t)b.n * l.planes * l.plane_rows);
+  if (save)
+    hipLaunchKernelGGL(fp8_save_generic<kScaleBf16>, dim3(grid), dim3(kThreads), 0, stream, (const uint16_t*)pool, g,
+                       b);
+  else
+    hipLaunchKernelGGL(fp8_restore_generic<kScaleBf16>, dim3(grid), dim3(kThreads), 0, stream, (uint16_t*)pool, g, b);
+  return hipGetLastError();
 }
 
 template <bool kTokens>
@@ -1153,27 +1167,29 @@ static hipError_t launch_raw(bool to_entry, void* pool, const kvx_block_layout& 
   const int64_t plane_bytes = (int64_t)l.plane_rows * l.head_dim * l.elem_bytes;
   if (entry_plane_stride < 0) entry_plane_stride = plane_bytes;
   if (last_bytes < 0) last_bytes = plane_bytes;
-  const bool vec = access == kVectorAccess && plane_bytes % 16 == 0 && entry_plane_stride % 16 == 0 && last_bytes % 16 == 0;
+  const bool vec = access == kVectorAccess && plane_bytes % 16 == 0 && entry_plane_stride % 16 == 0 &&
+                   last_bytes % 16 == 0;
   const int64_t es = l.elem_bytes;
   if (vec) {
     PlaneGeom g = make_geom(l, 0);
-    if (max_grid > 0) {
-      if ((unsigned)max_grid < set_tiles(g, b.n, kTokens, plane_bytes, last_bytes, kThreads * kStrideCopyVecs * 16)) {
-        if (to_entry)
-          hipLaunchKernelGGL((raw_copy_kernel<true, true, kTokens, kOrderDispatch>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
-                             (uint8_t*)pool, g, b, plane_bytes, es, entry_plane_stride, last_bytes);
-        else
-          hipLaunchKernelGGL((raw_copy_kernel<false, true, kTokens, kOrderDispatch>), dim3((unsigned)max_grid), dim3(kThreads), 0, stream,
-                             (uint8_t*)pool, g, b, plane_bytes, es, entry_plane_stride, last_bytes);
+    if constexpr (!kTokens) {
+      const unsigned cap = (unsigned)std::max(max_grid, 0);
+      if (cap > 0 && cap < set_tiles(g, b.n, false, plane_bytes, last_bytes, kThreads * kStrideCopyVecs * 16)) {
+        auto kernel = to_entry ? raw_copy_kernel<true, true, false, kOrderDispatch>
+                               : raw_copy_kernel<false, true, false, kOrderDispatch>;
+        hipLaunchKernelGGL(kernel, dim3(cap), dim3(kThreads), 0, stream, (uint8_t*)pool, g, b, plane_bytes, es,
+                           entry_plane_stride, last_bytes);
         return hipGetLastError();
       }
     }
     const unsigned grid = set_tiles(g, b.n, kTokens, plane_bytes, last_bytes, kCopyThreads * kCopyVecs * 16);
-    constexpr int kRuns = kTokens ? kTokenCopyOrder : kCopyOrder;
-    auto kernel = grid < kCopyRunTiles ? (to_entry ? raw_copy_kernel<true, false, kTokens, kOrderDispatch>
-                                                   : raw_copy_kernel<false, false, kTokens, kOrderDispatch>)
-                                       : (to_entry ? raw_copy_kernel<true, false, kTokens, kRuns>
-                                                   : raw_copy_kernel<false, false, kTokens, kRuns>);
+    auto kernel = to_entry ? raw_copy_kernel<true, false, kTokens, kOrderDispatch>
+                           : raw_copy_kernel<false, false, kTokens, kOrderDispatch>;
+    if constexpr (!kTokens) {
+      if (grid >= kCopyRunTiles)
+        kernel = to_entry ? raw_copy_kernel<true, false, false, kCopyOrder>
+                          : raw_copy_kernel<false, false, false, kCopyOrder>;
+    }
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kCopyThreads), 0, stream, (uint8_t*)pool, g, b, plane_bytes, es,
                        entry_plane_stride, last_bytes);
   } else {
@@ -1230,6 +1246,7 @@ bool striding_restore_supported(const kvx_block_layout& l, int32_t format, Acces
 hipError_t launch_restore(void* pool, const kvx_block_layout& l, int32_t format, const BlockBatch& b,
                           int64_t scale_offset, Access access, int32_t max_grid, hipStream_t stream) {
   if (b.n <= 0) return hipSuccess;
+  if (max_grid > 0 && !striding_restore_supported(l, format, access)) return hipErrorInvalidValue;
   if (format == KVX_FORMAT_RAW) return launch_raw<false>(false, pool, l, b, access, -1, -1, max_grid, stream);
   return l.scale_dtype == KVX_SCALE_BF16
              ? launch_fp8<true, false>(false, pool, l, b, scale_offset, access, max_grid, stream)
