@@ -10,6 +10,10 @@ from kvx import _lib, ops
 pytestmark = pytest.mark.gpu
 
 
+class Subclass(torch.Tensor):
+    pass
+
+
 class Declines:
     """Stands in for the binding and takes no call, so the Python checks run."""
 
@@ -69,6 +73,11 @@ def test_the_binding_takes_the_usual_calls(gpu):
     slots = torch.zeros(4, dtype=torch.int32, device=gpu)
     assert bind.store(key, key, pool[0, 0], pool[1, 0], slots) == 0
     # Subclasses, other sequences and other integers are left to Python.
+    sub = pool.as_subclass(Subclass)
+    assert bind.store(key.as_subclass(Subclass), key, pool[0, 0], pool[1, 0], slots) is None
+    assert bind.codec(True, source.as_subclass(Subclass), payload, torch.empty((*source.shape[:-1], 1), device=gpu)) is None
+    assert bind.blocks(True, sub, [1], [staging.data_ptr()], ops.FORMAT_RAW, None) is None
+    ops.save_blocks(sub, [1], [staging.data_ptr()], ops.FORMAT_RAW)
     assert bind.store(key, key, pool[0, 0], pool[1, 0], slots.long()) is None
     assert bind.store(key[:0], key[:0], pool[0, 0], pool[1, 0], slots[:0]) is None
     assert bind.blocks(True, pool, iter([1]), [staging.data_ptr()], ops.FORMAT_RAW, None) is None

@@ -118,7 +118,8 @@ def make_pool(device, layers=4, blocks=12, bs=256, heads=8, hd=128, seed=0):
     return (t / chi.add_(1e-3).sqrt() * 0.5).to(torch.bfloat16)
 
 
-# The vector kernels cover head_dim 64, 128 and 256 in tiles of 4-16 rows; the
+# The tiled kernels cover head_dim 128 and 256, and small saves of 64, in tiles
+# of 4-16 rows; other rows of whole 8-element pieces run the linear kernels. The
 # last three geometries leave a ragged last tile in every plane (15, 7 and 6 rows).
 # heads=1, hd=128 is one tensor-parallel rank's share of Qwen3-8B at TP=8.
 @pytest.mark.parametrize("geometry", [dict(), dict(layers=2, blocks=6, bs=256, heads=1, hd=4),
