@@ -58,6 +58,58 @@ def test_fp8_blocks_of_any_row_width(gpu, layers, bs, heads, hd, scale_dtype, sh
     assert np.array_equal(after, before)
 
 
+# The linear kernels: rows of 1 to 24 pieces, and payloads on 8 bytes only, in small launches (2 x 96 rows) and in
+# launches of more than 196,608 pieces.
+@pytest.mark.parametrize("scale_dtype", SCALES)
+@pytest.mark.parametrize("hd,shift,rows", [(64, 8, 96), (64, 0, 20100), (96, 0, 96), (96, 0, 10100), (80, 0, 10100),
+                                           (112, 0, 10100), (192, 0, 10100), (8, 0, 96), (8, 0, 100100),
+                                           (128, 8, 96), (128, 8, 10100)])
+def test_fp8_rows_with_nan_or_infinity_of_any_width(gpu, hd, shift, rows, scale_dtype):
+    fp32 = scale_dtype == torch.float32
+    bits = finite_bf16_rows(2 * rows, hd, seed=hd)
+    rng = np.random.default_rng(rows)
+    kinds = np.zeros(2 * rows, dtype=np.int32)  # of every third row: 1 a NaN, 2 an infinity, 3 both, 4 the lowest value
+    kinds[::3] = rng.integers(1, 5, size=kinds[::3].size)
+    at, other = rng.integers(0, hd, size=(2, 2 * rows))
+    other = np.where(other == at, (at + 1) % hd, other)
+    nans = rng.choice(np.array([0x7FC0, 0xFFC0, 0x7F81, 0xFFFF], dtype=np.uint16), size=2 * rows)
+    infinities = rng.choice(np.array([0x7F80, 0xFF80], dtype=np.uint16), size=2 * rows)
+    for kind, first, second in ((1, nans, None), (2, infinities, None), (3, infinities, nans),
+                                (4, np.full(2 * rows, 0xFF7F, dtype=np.uint16), None)):
+        i = np.flatnonzero(kinds == kind)
+        bits[i, at[i]] = first[i]
+        if second is not None:
+            bits[i, other[i]] = second[i]
+    pool = bf16_tensor(bits, gpu).view(2, 1, 1, rows, 1, hd)
+    _, offset, stride = ops.entry_layout(ops.pool_layout(pool, scale_dtype), ops.FORMAT_FP8)
+    staging = torch.zeros(stride + 256, dtype=torch.uint8, device=gpu)
+    entry = [staging.data_ptr() + shift]
+    ops.save_blocks(pool, [0], entry, ops.FORMAT_FP8, scale_dtype)
+    back = torch.zeros_like(pool)
+    ops.restore_blocks(back, [0], entry, ops.FORMAT_FP8, scale_dtype)
+    staged, back = u8(staging), bf16_bits(back).reshape(2 * rows, hd)
+    codes = staged[shift:shift + 2 * rows * hd].reshape(2 * rows, hd)
+    scales = staged[shift + offset:shift + offset + 2 * rows * (4 if fp32 else 2)].copy()
+    scales = scales.view(np.float32) if fp32 else (scales.view(np.uint16).astype(np.uint32) << 16).view(np.float32)
+
+    finite = (kinds == 0) | (kinds == 4)
+    want_codes, want_scales = oracle.quantize(bits[finite], fp32)
+    assert np.array_equal(codes[finite], want_codes)
+    want_back = oracle.dequantize(want_codes, want_scales, fp32)
+    assert np.array_equal(back[finite], want_back)
+    want_scales = want_scales.ravel()
+    want_scales = want_scales if fp32 else (want_scales.view(np.uint16).astype(np.uint32) << 16).view(np.float32)
+    assert np.array_equal(scales[finite], want_scales)
+    nan, infinite = (kinds == 1) | (kinds == 3), kinds == 2
+    assert np.isnan(scales[nan]).all() and np.isposinf(scales[infinite]).all()
+    assert ((codes[nan] & 0x7F) == 0x7F).all()
+    # Finite values over an infinite scale are signed zeros; infinity over infinity is NaN.
+    is_inf = (bits[infinite] & 0x7FFF) == 0x7F80
+    assert ((codes[infinite][is_inf] & 0x7F) == 0x7F).all()
+    assert np.array_equal(codes[infinite][~is_inf], (bits[infinite][~is_inf] >> 8 & 0x80).astype(np.uint8))
+    assert ((back[~finite] & 0x7FFF) > 0x7F80).all()  # NaN times anything, and zero times infinity
+
+
 # Token counts whose planes of scales (and, with 3 heads of 40, of codes) are not multiples of 16 bytes.
 @pytest.mark.parametrize("scale_dtype", SCALES)
 @pytest.mark.parametrize("heads,hd,tokens", [(1, 128, 1), (1, 128, 257), (2, 128, 511), (1, 64, 513), (3, 40, 301),
@@ -161,15 +213,18 @@ def test_store_kvcache_of_any_row_width(gpu, heads, hd, tokens):
 
 
 def test_store_kvcache_beyond_one_launch(gpu):
-    # More than 2^30 16-byte pieces take several launches. One row expanded over every token; few slots are real.
-    row = torch.randn((1, 8, 128), device=gpu).to(torch.bfloat16)
+    # More than 2^30 16-byte pieces take several launches. Rows overlap: key's are 8 elements apart and value's 16, so
+    # every token has its own, in K and in V; few slots are real.
     tokens = (1 << 22) + 3
+    g = torch.Generator(device=gpu).manual_seed(1)
+    key, value = (torch.randn(tokens * step + 1024, generator=g, device=gpu, dtype=torch.bfloat16)
+                  .as_strided((tokens, 8, 128), (step, 128, 1)) for step in (8, 16))
     slots = torch.full((tokens,), -1, dtype=torch.int32, device=gpu)
-    where = torch.tensor([0, (1 << 22) - 1, 1 << 22, tokens - 1], device=gpu)
-    slots[where] = torch.tensor([5, 0, 7, 3], dtype=torch.int32, device=gpu)
+    where = [0, (1 << 22) - 1, 1 << 22, tokens - 1]
+    slots[torch.tensor(where, device=gpu)] = torch.tensor([5, 0, 7, 3], dtype=torch.int32, device=gpu)
     caches = torch.zeros((2, 1, 8, 8, 128), dtype=torch.bfloat16, device=gpu)
-    ops.store_kvcache(row.expand(tokens, 8, 128), row.expand(tokens, 8, 128), caches[0], caches[1], slots)
-    for cache in caches:
-        for slot in range(8):
-            want = row[0] if slot in (0, 3, 5, 7) else torch.zeros_like(row[0])
-            assert torch.equal(cache[0, slot], want), slot
+    ops.store_kvcache(key, value, caches[0], caches[1], slots)
+    expect = torch.zeros_like(caches)
+    for token, slot in zip(where, [5, 0, 7, 3]):
+        expect[0, 0, slot], expect[1, 0, slot] = key[token], value[token]
+    assert torch.equal(caches.view(torch.int16), expect.view(torch.int16))
