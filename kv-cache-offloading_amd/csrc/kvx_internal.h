@@ -23,8 +23,12 @@ struct BlockBatch {
 // 2^l >= d and mul = floor(2^(31 + l) / d) + 1, mul * d exceeds 2^(31 + l) by at
 // most d <= 2^l, so n times that excess stays below 2^(31 + l) and the quotient
 // is exact. mul < 2^33 / 2 fits 32 bits. The kernels find a tile's entry and
-// plane by it: two integer divisions ahead of a workgroup's first load took the
-// save of 128 Qwen3-8B blocks from 1,092 to 1,125 us on MI355X.
+// plane by it, ahead of a workgroup's first load. With two integer divisions
+// instead, measured on MI355X on one card (us): FP8 saves of 128 / 48 / 16 / 1
+// Qwen3-8B blocks 1108 / 466 / 141.1 / 12.2, 1092 / 436 / 137.2 / 11.7 so;
+// their restores 1139.5 and 1139.1 for 128 blocks, 12.6 and 12.4 for one; BF16
+// copies of 32 Qwen3-0.6B blocks 562 and 560, but of 4 Qwen3-8B ones 92.2 and
+// 92.8.
 struct FastDiv {
   uint32_t mul;
   uint32_t shift;

@@ -157,10 +157,10 @@ constexpr int kCopyOrder = 9;
 // 20,000 tokens, 172 / 175 / 184.
 constexpr int kTokenRestoreRuns = 8;
 constexpr int64_t kTokenRunPlane = 256 << 10;  // elements of a block's plane
-// Smaller copies leave no whole number of run rounds and keep the dispatcher's
-// order: 147,456 tiles (4 Qwen3-8B blocks each way) 98.4 us, 99.2 in runs of
-// 512; 294,912 tiles 184.0 and 181.9; 64 blocks of 72 x 1024 rows of 128
-// (1.18 M tiles) 936 and 757.
+// Smaller copies keep the dispatcher's order. The line is a measured crossover:
+// 147,456 tiles (4 Qwen3-8B blocks each way) 98.4 us, 99.2 in runs of 512;
+// 294,912 tiles 184.0 and 181.9; 64 blocks of 72 x 1024 rows of 128 (1.18 M
+// tiles) 936 and 757.
 constexpr unsigned kCopyRunTiles = 192 << 10;
 
 // ---------------------------------------------------------------------------
@@ -492,8 +492,8 @@ __global__ __launch_bounds__(kBlock) void fp8_restore_kernel(uint16_t* __restric
     if (row < rows) s = scale_value_host(host_rsrc(scales, (int64_t)rows * (kScaleBf16 ? 2 : 4)), row, kScaleBf16);
   } else {
     // The scales' place before or after the codes' loads is measured: fp32 first
-    // (16 blocks 147.0 us, after 148.2; 30 blocks of 4 x 256 293 and 299.5),
-    // bf16 after (64 blocks 582, first 596; 16 blocks of one KV head 22.0, 22.8).
+    // (128 blocks 1130 us, after 1133; 64 591 and 595; 16 140.7 and 140.8), bf16
+    // after (64 blocks 582, first 596; 16 blocks of one KV head 22.0, 22.8).
     if (!kScaleBf16 && row < rows) s = scale_value(scales, row, false);
     for (int i = threadIdx.x; i < kPieces; i += kBlock)
       codes[i] = tc.row0 + i * 16 / kHd < rows ? load_nt16(tile_codes + i * 16) : make_uint4(0, 0, 0, 0);
@@ -777,6 +777,13 @@ __global__ __launch_bounds__(kThreads) void raw_copy_generic(uint8_t* __restrict
 // (5.5 before); 8,192 tokens of 32 heads x 96 34.3 (one workgroup per token and
 // 2-byte pieces before: 51.5). No faster: loading the row before its slot is
 // known. Slower: two pieces per thread, of one row (25.8) or K and V (25.9).
+// In a model step K and V were just written. Behind a fused QKV product and the
+// rotary embedding, 64 / 128 / 256 threads / the kernel before: 4,096 tokens in
+// paged blocks 6.4 / 6.2 / 6.9 / 6.4, 8,192 13.8 / 13.8 / 14.9 / 17.8, 16,384
+// 23.5 / 25.8 / 26.4 / 28.6; 16,384 of 2 heads 8.3 / 8.3 / 8.2 / 9.1. Only where
+// every token reads the same cached row, which no step does, is the dispatch of
+// one-wave workgroups (4.5 per ns) the bound: 16,384 tokens 16.7 / 11.3 / 11.6 /
+// 11.9.
 constexpr int kStoreThreads = 64;
 // Small batches are launched and ramped up faster by larger workgroups. The
 // two sizes cross between 524,288 pieces (1 head x 128, 16,384 tokens: 5.3 us
@@ -1272,7 +1279,7 @@ hipError_t launch_store_kvcache(const void* key, int64_t key_stride, const void*
                        ks % 16 == 0 && vs % 16 == 0 && row_bytes % 16 == 0;
   const int64_t row16 = row_bytes / 16;
   if (aligned && 2 * row16 <= kStoreMostPieces) {
-    // Launches of at most kStoreMostPieces pieces (32 GiB of rows).
+    // Launches of at most kStoreMostPieces pieces (16 GiB of rows).
     const int64_t most = kStoreMostPieces / (2 * row16);
     for (int64_t first = 0; first < n; first += most) {
       const int64_t count = std::min(most, n - first), pieces = count * 2 * row16;
