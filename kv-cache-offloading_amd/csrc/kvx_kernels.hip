@@ -996,38 +996,44 @@ constexpr int kLinearSaveVecs = 3;
 constexpr int kLinearRestoreBlock = 256;
 constexpr int kLinearRestoreVecs = 2;
 constexpr int kLinearMaxPieces = kLinearSaveBlock * kLinearSaveVecs;  // a row must fit a save tile
-// Small planes and small launches take one-wave workgroups with fewer pieces
-// per thread. A launch of many planes is bound by dispatch, which starts four
-// of these for one of 256 threads, and a small launch by the latency of one
-// workgroup, its barriers and its memory passes. Measured on MI355X (us, in a
-// captured graph), workgroups of 256 threads / of one wave:
+// Many small planes, and small launches of larger ones, take one-wave
+// workgroups with fewer pieces per thread. A launch of many planes is bound by
+// dispatch, which starts four of these for one of 256 threads, and a small
+// launch by the latency of one workgroup, its barriers and its memory passes.
+// Measured on MI355X (us, in a captured graph), workgroups of 256 threads / of
+// one wave:
 // - 16,384 planes of 8 rows of 64: save 15.3 / 7.5, restore 13.4 / 6.9; of one
-//   row of 96: 14.9 / 6.2 and 13.1 / 5.6;
+//   row of 96: 14.9 / 6.2 and 13.1 / 5.6; 1,024 of 8 rows of 64: 2.9 / 2.5 and
+//   2.5 / 2.2; but 516 of 17 rows of 64: 2.9 / 3.1 and 2.35 / 2.45;
 // - planes of 192 pieces (4,608 of 16 rows of 96): save 7.3 / 6.9, restore 6.65
 //   / 6.4; of 256 pieces (4,096 of 32 rows of 64): 7.3 / 5.9 but 6.7 / 6.8;
-// - one plane of 24,500 rows of 64 (196,000 pieces): save 3.7 / 3.4, restore
-//   3.2 / 3.15; of 32,768 (262,144): 3.95 / 3.55 but 3.45 / 3.6.
+// - one plane of 200 pieces (a piece per thread in one workgroup): save 2.0 /
+//   2.3; of 400 2.4 / 2.3; of 24,500 rows of 64 (196,000 pieces): 3.7 / 3.4 and
+//   restored 3.2 / 3.15; of 32,768 (262,144): 3.95 / 3.55 but 3.45 / 3.6.
 // Token copies keep the larger ones: 17 tokens of 72 planes of one head of 64
 // gathered in 2.3 us, 2.7 with one wave.
 constexpr int kLinearSmallBlock = 64;
 constexpr int kLinearSmallSaveVecs = 2;
 constexpr int kLinearSmallRestoreVecs = 1;
 constexpr int64_t kLinearSmallPlane = 192;
+constexpr int64_t kLinearManyPlanes = 1024;
 constexpr int64_t kLinearSmallTotal = 192 << 10;
 // Saves of rows of 64 up to here are latency-bound and stay with the tiled
 // kernel, whose row maxima need no barrier: 2,048 rows 2.4 us (2.7 with the
-// linear one), 4,096 2.75 (2.9), 8,200 3.0 (3.0).
+// linear one), 4,096 2.75 (2.9), 8,200 3.0 (3.0). Planes of up to 32 rows are
+// one piece per thread of a linear workgroup, which is faster: 720 of 3 rows
+// 2.75 us, 2.95 in tiles.
 constexpr int64_t kTiledSave64Rows = 8192;
 constexpr int kLinePieces = 16;  // 128 bytes of codes
 
 // Tiles of at most `most` items (a multiple of `step`) for a plane of `items`: of that size, unless the last one
-// would then be less than a quarter full, and of about equal size, in steps of `step`, if so. A nearly empty tile
-// costs almost a full one: 4,096 planes of 65 rows of 64 (520 pieces) restored in 15.5 us as 512 + 8, 12.1 us as
-// 272 + 248; 2,048 of 97 saved in 12.1 us as 96 + 1 rows, 9.5 as 50 + 47. Planes whose last tile is fuller gained
-// nothing (96 rows of 96 restored: 23.8 and 24.1).
-static int64_t spread(int64_t items, int64_t most, int64_t step) {
+// would then be at most 1/part full, and of about equal size, in steps of `step`, if so. A nearly empty tile costs
+// almost a full one: 4,096 planes of 65 rows of 64 (520 pieces) restored in 15.5 us as 512 + 8, 12.1 us as 272 + 248;
+// 2,048 of 97 saved in 12.1 us as 96 + 1 rows, 9.5 as 50 + 47, of 120 12.5 and 10.6. With fuller last tiles restores
+// lost (a fifth: 512 planes of 141 rows of 64 4.65 us, 4.85 spread; a quarter: 4,096 of 96 rows of 96 23.8 and 24.1).
+static int64_t spread(int64_t items, int64_t most, int64_t step, int64_t part) {
   const int64_t last = items % most;
-  if (items <= most || last == 0 || last * 4 >= most) return most;
+  if (items <= most || last == 0 || last * part > most) return most;
   const int64_t tiles = items / most + 1, even = (items + tiles - 1) / tiles;
   return (even + step - 1) / step * step;
 }
@@ -1052,7 +1058,8 @@ static hipError_t launch_fp8_linear_as(bool save, void* pool, const kvx_block_la
   if (!save) {
     constexpr int kPieces = kRestoreBlock * kRestoreVecs;
     PlaneGeom g = make_geom(l, scale_offset, span);
-    const int64_t pieces = (int64_t)g.plane_rows * row_pieces, tile = spread(pieces, kPieces, kLinePieces);
+    const int64_t pieces = (int64_t)g.plane_rows * row_pieces;
+    const int64_t tile = spread(pieces, kPieces, kLinePieces, 8);
     const unsigned grid = set_tiles(g, b.n, kTokens, pieces, (int64_t)g.last_rows * row_pieces, tile);
     hipLaunchKernelGGL((fp8_restore_linear<kRestoreBlock, kRestoreVecs, kScaleBf16, kTokens>), dim3(grid),
                        dim3(kRestoreBlock), 0, stream, (uint16_t*)pool, g, (int)tile, row_of, b);
@@ -1061,7 +1068,7 @@ static hipError_t launch_fp8_linear_as(bool save, void* pool, const kvx_block_la
   // As many rows as fit, in whole 128-byte lines of codes (and of bf16) if any such number fits.
   const int32_t most = kSaveBlock * kSaveVecs / row_pieces;
   const int32_t lines = 128 / std::min(128, l.head_dim & -l.head_dim);
-  const int32_t rows = most >= lines ? (int32_t)spread(l.plane_rows, most / lines * lines, lines) : most;
+  const int32_t rows = most >= lines ? (int32_t)spread(l.plane_rows, most / lines * lines, lines, 4) : most;
   PlaneGeom g = make_geom(l, scale_offset, span);
   const unsigned grid = set_tiles(g, b.n, kTokens, g.plane_rows, g.last_rows, rows);
   if constexpr (!kTokens) {
@@ -1082,8 +1089,10 @@ static hipError_t launch_fp8_linear(bool save, void* pool, const kvx_block_layou
                                     int64_t scale_offset, int32_t max_grid, hipStream_t stream,
                                     const TokenSpan* span) {
   const int64_t row = l.head_dim / 8, plane = row * l.plane_rows;
+  const int64_t planes = (int64_t)l.planes * b.n;
   if (!kTokens && max_grid <= 0 && row <= kLinearSmallBlock * kLinearSmallSaveVecs &&
-      (plane <= kLinearSmallPlane || plane * l.planes * b.n <= kLinearSmallTotal))
+      (plane <= kLinearSmallPlane ? planes >= kLinearManyPlanes
+                                  : plane > kLinearSaveBlock && plane * planes <= kLinearSmallTotal))
     return launch_fp8_linear_as<kLinearSmallBlock, kLinearSmallSaveVecs, kLinearSmallBlock, kLinearSmallRestoreVecs,
                                 kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
   return launch_fp8_linear_as<kLinearSaveBlock, kLinearSaveVecs, kLinearRestoreBlock, kLinearRestoreVecs, kScaleBf16,
@@ -1155,7 +1164,7 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
   // kernels and small saves are used. The linear kernels restore 100 blocks of
   // 64 x 1024 such rows in 210 us (245 in tiled ones) and save them in 201 us (242).
   if constexpr (!kTokens) {
-    const bool small_save = save && (int64_t)b.n * l.planes * l.plane_rows <= kTiledSave64Rows;
+    const bool small_save = save && (int64_t)b.n * l.planes * l.plane_rows <= kTiledSave64Rows && l.plane_rows > 32;
     if (access == kVectorAccess && l.head_dim == 64 && (max_grid > 0 || small_save))
       return launch_fp8_tiled<64, 1, kScaleBf16, false>(save, pool, l, b, scale_offset, max_grid, stream, span);
   }

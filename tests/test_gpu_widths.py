@@ -24,11 +24,14 @@ def finite_pool(gpu, layers, blocks, bs, heads, hd, seed=0):
 WIDTHS = [(2, 63, 1, 96), (2, 64, 1, 96), (1, 65, 1, 96), (1, 256, 3, 96), (2, 73, 1, 80), (1, 49, 2, 112),
           (2, 33, 1, 192), (1, 300, 5, 8), (1, 97, 1, 16), (1, 77, 1, 40), (1, 3, 1, 6144), (1, 2, 1, 6152),
           (1, 5, 3, 100), (2, 49, 1, 128), (1, 17, 1, 256), (1, 200, 1, 64)]
-# The launches above are small ones, in one-wave workgroups of 128 pieces to save and 64 to restore (at most 196,608
-# pieces, here in 2 blocks). Larger: planes at and around whole tiles, a last tile spread over the others (65 and 97
-# rows of 64, 65 of 96, 800 of 8) and not (81 of 96), planes of at most 192 pieces (one wave again) and just above.
+# The launches above are small ones: in one-wave workgroups of 128 pieces to save and 64 to restore where planes have
+# more than 256 pieces. Launches of more than 196,608 pieces: planes at and around whole tiles, a last tile spread over
+# the others (97 rows of 64, 65 of 96 and 800 of 8 to save, 65 of 64 to restore) and not (81 of 96). 1,040 planes of 192
+# pieces (one wave again) and of 200, and 1,000 of 192.
 WIDTHS += [(66, 64, 1, 96), (66, 65, 1, 96), (60, 81, 1, 96), (100, 65, 1, 64), (66, 97, 1, 64), (66, 800, 1, 8),
-           (260, 24, 1, 64), (260, 25, 1, 64), (250, 16, 1, 96)]
+           (260, 24, 1, 64), (260, 25, 1, 64), (260, 16, 1, 96), (250, 16, 1, 96)]
+# Rows of 64 around the tiled kernel's 32 rows a plane to save.
+WIDTHS += [(2, 32, 1, 64), (2, 33, 1, 64)]
 # Rows of 64 above the tiled kernel's 8,192 rows to save. Many planes of a few narrow rows (above 8,192 per 8 elements
 # of the row), which one thread per row handles, and the same with a row more.
 WIDTHS += [(16, 130, 1, 64), (2060, 8, 1, 8), (2060, 9, 1, 8), (2060, 10, 1, 8), (4110, 2, 1, 16), (4110, 3, 1, 16)]
@@ -152,7 +155,7 @@ def test_raw_tokens_of_any_count_and_width(gpu, heads, hd, tokens):
 
 
 @pytest.mark.parametrize("scale_dtype", SCALES)
-@pytest.mark.parametrize("heads,hd", [(3, 96), (1, 80)])
+@pytest.mark.parametrize("heads,hd", [(3, 96), (1, 80), (2, 64), (64, 64)])
 def test_engine_saves_and_restores_of_other_widths(gpu, heads, hd, scale_dtype):
     # Saves of 1-2 blocks behind a busy caller are written to the host slots by a capped grid of workgroups.
     from kvx.engine.cpu_prefix_cache import _CopyEngine
