@@ -593,10 +593,11 @@ __global__ __launch_bounds__(kBlock) void fp8_save_linear(const uint16_t* __rest
 template <int kBlock, int kVecs, bool kScaleBf16, bool kTokens>
 __global__ __launch_bounds__(kBlock) void fp8_restore_linear(uint16_t* __restrict__ pool, PlaneGeom g,
                                                             int tile_pieces, FastDiv row_of, BlockBatch b) {
+  if (kTokens) tile_pieces = kBlock * kVecs;
   // row0 counts pieces here.
   const TileCoord tc = tile_coord<kTokens, kTokens ? kTokenRestoreOrder : kRestoreOrder>(g, tile_pieces);
   int pieces = (tc.entry == b.n - 1 ? g.last_rows : g.plane_rows) * (g.head_dim / 8);
-  pieces = min(pieces, tc.row0 + tile_pieces);
+  if (!kTokens) pieces = min(pieces, tc.row0 + tile_pieces);
   uint16_t* dst = pool + (int64_t)b.ids[tc.entry] * g.block_stride + (int64_t)tc.plane * g.plane_stride;
   const uint8_t* payload =
       reinterpret_cast<const uint8_t*>(b.entries[tc.entry]) + (int64_t)tc.plane * g.payload_plane_stride;
@@ -953,15 +954,19 @@ __global__ void zero_counters(uint64_t* c) {
 // Launchers
 
 // Tiles of `tile` items for the batch's planes of `items`, and of `last_items` in its last entry; the launch's tiles.
-// Those of a plane of token entries are rounded up to whole rounds of the 8 XCDs, if the last entry has room for the
-// empty ones: each XCD then writes the same share of every 8 tiles in all planes. Without, scatters took up to 13%
-// longer (2,049 tokens of one head of 128 12.7 us, 11.3 with; 20,001 of 2 heads 175.9 and 174.8).
+// Those of a large plane of token entries are rounded up to whole rounds of the 8 XCDs, if the last entry has room for
+// the empty ones: each XCD then writes the same share of every 8 tiles in all planes. Without, scatters took up to 13%
+// longer (2,049 tokens of one head of 128, 257 tiles, 12.7 us, 11.3 with; 20,001 of 2 heads 175.9 and 174.8). In small
+// planes the first XCDs would get all the work instead (17 tokens of one head of 128, 2 tiles, gathered in 3.0 us, 3.5
+// rounded); around the line the two are equal (1,001 tokens of one head, 126 tiles, scattered in 6.8 both ways).
+constexpr int64_t kTokenRoundTiles = 128;
 static unsigned set_tiles(PlaneGeom& g, int32_t n, bool tokens, int64_t items, int64_t last_items, int64_t tile) {
   g.chunks = (int32_t)((items + tile - 1) / tile);
   g.inner_of = FastDiv((uint32_t)g.chunks);
   if (tokens) {
     const int64_t tiles = (int64_t)(n - 1) * g.chunks + (last_items + tile - 1) / tile;
-    g.outer_tiles = (int32_t)std::min((int64_t)n * g.chunks, (tiles + 7) / 8 * 8);
+    const int64_t rounds = tiles < kTokenRoundTiles ? tiles : (tiles + 7) / 8 * 8;
+    g.outer_tiles = (int32_t)std::min((int64_t)n * g.chunks, rounds);
   } else {
     g.outer_tiles = g.planes * g.chunks;
   }
@@ -1059,7 +1064,7 @@ static hipError_t launch_fp8_linear_as(bool save, void* pool, const kvx_block_la
     constexpr int kPieces = kRestoreBlock * kRestoreVecs;
     PlaneGeom g = make_geom(l, scale_offset, span);
     const int64_t pieces = (int64_t)g.plane_rows * row_pieces;
-    const int64_t tile = spread(pieces, kPieces, kLinePieces, 8);
+    const int64_t tile = kTokens ? kPieces : spread(pieces, kPieces, kLinePieces, 8);
     const unsigned grid = set_tiles(g, b.n, kTokens, pieces, (int64_t)g.last_rows * row_pieces, tile);
     hipLaunchKernelGGL((fp8_restore_linear<kRestoreBlock, kRestoreVecs, kScaleBf16, kTokens>), dim3(grid),
                        dim3(kRestoreBlock), 0, stream, (uint16_t*)pool, g, (int)tile, row_of, b);
@@ -1163,10 +1168,11 @@ static hipError_t launch_fp8(bool save, void* pool, const kvx_block_layout& l, c
   // Rows of 64 fill half of a restore wave's code loads: only their striding
   // kernels and small saves are used. The linear kernels restore 100 blocks of
   // 64 x 1024 such rows in 210 us (245 in tiled ones) and save them in 201 us (242).
-  if constexpr (!kTokens) {
-    const bool small_save = save && (int64_t)b.n * l.planes * l.plane_rows <= kTiledSave64Rows && l.plane_rows > 32;
-    if (access == kVectorAccess && l.head_dim == 64 && (max_grid > 0 || small_save))
-      return launch_fp8_tiled<64, 1, kScaleBf16, false>(save, pool, l, b, scale_offset, max_grid, stream, span);
+  if (access == kVectorAccess && l.head_dim == 64) {
+    const int64_t last = span ? span->last_rows : l.plane_rows, rows = (b.n - 1) * (int64_t)l.plane_rows + last;
+    const bool small_save = save && l.planes * rows <= kTiledSave64Rows && (b.n > 1 ? l.plane_rows : last) > 32;
+    if (max_grid > 0 || small_save)
+      return launch_fp8_tiled<64, 1, kScaleBf16, kTokens>(save, pool, l, b, scale_offset, max_grid, stream, span);
   }
   // Other widths, and payloads on 8 bytes only: the linear kernels. They
   // take rows of 128 and 256 too, but save 128 Qwen3-8B blocks in 1,131 us

@@ -120,7 +120,9 @@ def test_fp8_rows_with_nan_or_infinity_of_any_width(gpu, hd, shift, rows, scale_
                                              # the last block at, above and below whole tiles
                                              (1, 128, 16), (1, 128, 273), (1, 256, 264), (1, 64, 352), (1, 96, 64),
                                              # planes scattered in runs of tiles per XCD
-                                             (8, 128, 700), (4, 256, 300)])
+                                             (8, 128, 700), (4, 256, 300),
+                                             # rows of 64 above and below the tiled kernel's launches and planes
+                                             (8, 64, 600), (1, 64, 32), (1, 64, 33), (4, 64, 257)])
 def test_fp8_tokens_of_any_count_and_width(gpu, heads, hd, tokens, scale_dtype):
     pool = finite_pool(gpu, 2, 6, 256, heads, hd, seed=tokens)
     before = bf16_bits(pool)
@@ -140,7 +142,7 @@ def test_fp8_tokens_of_any_count_and_width(gpu, heads, hd, tokens, scale_dtype):
 
 # A tile is 1 KiB of a plane: the last block's share a fraction of one, whole ones, and one row more or less.
 @pytest.mark.parametrize("heads,hd,tokens", [(1, 128, 1), (1, 128, 4), (1, 128, 259), (1, 128, 260), (1, 128, 261),
-                                             (3, 40, 301), (2, 256, 512), (1, 8, 320)])
+                                             (3, 40, 301), (2, 256, 512), (1, 8, 320), (1, 128, 521)])
 def test_raw_tokens_of_any_count_and_width(gpu, heads, hd, tokens):
     pool = finite_pool(gpu, 2, 6, 256, heads, hd, seed=tokens)
     before = bf16_bits(pool)
